@@ -63,7 +63,7 @@ kb_flux(const BItem* __restrict__ items, const BTile* __restrict__ tiles, int ax
     int i, j, k;
     if (!tile_thread(T, i, j, k)) return;
     const double* Pin = rk == 0 ? it.Pa : it.Pb;
-    flux_face<Law, Recon, Riem, R>(Pin, (R*)it.F[axis], it.G, axis, i, j, k, it.ctl);
+    flux_face<Law, Recon, Riem, R, -1>(Pin, (R*)it.F[axis], it.G, axis, i, j, k, it.ctl);
 }
 
 template <int Law, typename R, bool CT>

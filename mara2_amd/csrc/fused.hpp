@@ -84,11 +84,29 @@ __device__ __forceinline__ int periodic_index(const Geom& G, int a, int s)
     return min(max(s, 0), G.N[a] - 1);
 }
 
+// Flux through a face normal to axis AX from the states on its two sides:
+// hydro_state and hllc or hlle, by exact.hpp in binary64.
+template <int Riem, int AX, typename R>
+__device__ __forceinline__ void hydro_states_flux(const R* PL, const R* PR, R gamma, const exact::Gas& K, const R* n,
+                                                  R* F)
+{
+    if constexpr (sizeof(R) == 8) exact::face_flux<0, Riem, AX>(PL, PR, K, n, F);
+    else
+    {
+        State<R, 5> SL, SR;
+        hydro_state(gamma, PL, n, SL);
+        hydro_state(gamma, PR, n, SR);
+        if constexpr (Riem == 1) hllc(SL, SR, n, F);
+        else hlle<R, 5>(SL, SR, F);
+    }
+}
+
 // Flux through one face from a stencil of 2 NG zones per field (reference
 // IntercellFluxScheme + RiemannSolver, src/IntercellFluxSchemes.cpp:45-117).
-template <int Recon, int Riem, typename R>
+// AX: the face's axis, K the binary64 form's gas constants.
+template <int Recon, int Riem, int AX, typename R>
 __device__ __forceinline__ void hydro_face_flux(const R (&S)[5][2 * (Recon == 0 ? 1 : Recon == 1 ? 2 : 3)],
-                                                R theta, R gamma, const R* n, R* F)
+                                                R theta, R gamma, const exact::Gas& K, const R* n, R* F)
 {
     constexpr int NG = Recon == 0 ? 1 : Recon == 1 ? 2 : 3;
     R PL[5], PR[5];
@@ -111,11 +129,7 @@ __device__ __forceinline__ void hydro_face_flux(const R (&S)[5][2 * (Recon == 0 
             PR[q] = weno5<R, false>(S[q][1], S[q][2], S[q][3], S[q][4], S[q][5]);
         }
     }
-    State<R, 5> SL, SR;
-    hydro_state(gamma, PL, n, SL);
-    hydro_state(gamma, PR, n, SR);
-    if constexpr (Riem == 1) hllc(SL, SR, n, F);
-    else hlle<R, 5>(SL, SR, F);
+    hydro_states_flux<Riem, AX, R>(PL, PR, gamma, K, n, F);
 }
 
 // U = U(P0) of the binary32 flux form: p / (gamma - 1) of
@@ -149,6 +163,9 @@ k_fused_hydro(const double* __restrict__ Pin, const double* __restrict__ P0, dou
 
     if (!ctl->active) return;
     double dmin = 1.79769313486231570815e+308;  // this zone column's CFL minimum (last stage)
+    // binary64: the largest signal speed instead; division is monotone, so
+    // the smallest of the quotients Lmin / speed is that of the largest speed
+    double smax = 0.0;
     const int lane = threadIdx.x;
     const int row = threadIdx.y;
     const int tid = row * TX + lane;
@@ -168,6 +185,7 @@ k_fused_hydro(const double* __restrict__ Pin, const double* __restrict__ P0, dou
     const long long sxy = (long long)G.N[0] * G.N[1];
     const R theta = R(G.theta), gamma = R(G.gamma);
     const double igm1 = 1.0 / (G.gamma - 1.0);  // binary32 form's U(P0)
+    const exact::Gas K = exact::gas(G.gamma);   // binary64 form
     const R nx[3] = {R(G.nhat[0]), R(G.nhat[1]), R(G.nhat[2])};
     const R ny[3] = {R(G.nhat[3]), R(G.nhat[4]), R(G.nhat[5])};
     const R nz[3] = {R(G.nhat[6]), R(G.nhat[7]), R(G.nhat[8])};
@@ -192,7 +210,7 @@ k_fused_hydro(const double* __restrict__ Pin, const double* __restrict__ P0, dou
         for (int q = 0; q < 5; ++q)
 #pragma unroll
             for (int m = 0; m < 2 * NG; ++m) S[q][m] = W[q][m + 1];
-        hydro_face_flux<Recon, Riem, R>(S, theta, gamma, nz, Fzlo);
+        hydro_face_flux<Recon, Riem, 2, R>(S, theta, gamma, K, nz, Fzlo);
     }
 
     for (int k = kb; k < ke; ++k)
@@ -223,7 +241,7 @@ k_fused_hydro(const double* __restrict__ Pin, const double* __restrict__ P0, dou
             for (int q = 0; q < 5; ++q)
 #pragma unroll
                 for (int m = 0; m < 2 * NG; ++m) S[q][m] = W[q][m + 1];
-            if (cell_xy) hydro_face_flux<Recon, Riem, R>(S, theta, gamma, nz, Fzhi);
+            if (cell_xy) hydro_face_flux<Recon, Riem, 2, R>(S, theta, gamma, K, nz, Fzhi);
         }
         __syncthreads();
 
@@ -236,7 +254,7 @@ k_fused_hydro(const double* __restrict__ Pin, const double* __restrict__ P0, dou
             for (int q = 0; q < 5; ++q)
 #pragma unroll
                 for (int m = 0; m < 2 * NG; ++m) S[q][m] = plane[q][row + NG][lane + m];
-            hydro_face_flux<Recon, Riem, R>(S, theta, gamma, nx, Fx);
+            hydro_face_flux<Recon, Riem, 0, R>(S, theta, gamma, K, nx, Fx);
         }
         if (yface)
         {
@@ -245,7 +263,7 @@ k_fused_hydro(const double* __restrict__ Pin, const double* __restrict__ P0, dou
             for (int q = 0; q < 5; ++q)
 #pragma unroll
                 for (int m = 0; m < 2 * NG; ++m) S[q][m] = plane[q][row + m][lane + NG];
-            hydro_face_flux<Recon, Riem, R>(S, theta, gamma, ny, Fy);
+            hydro_face_flux<Recon, Riem, 1, R>(S, theta, gamma, K, ny, Fy);
 #pragma unroll
             for (int q = 0; q < 5; ++q) fy[q][row][lane] = Fy[q];
         }
@@ -262,7 +280,7 @@ k_fused_hydro(const double* __restrict__ Pin, const double* __restrict__ P0, dou
                     for (int q = 0; q < 5; ++q)
 #pragma unroll
                         for (int m = 0; m < 2 * NG; ++m) S[q][m] = plane[q][r + NG][TX + m];
-                    hydro_face_flux<Recon, Riem, R>(S, theta, gamma, nx, F);
+                    hydro_face_flux<Recon, Riem, 0, R>(S, theta, gamma, K, nx, F);
 #pragma unroll
                     for (int q = 0; q < 5; ++q) fxe[q][r] = F[q];
                 }
@@ -277,7 +295,7 @@ k_fused_hydro(const double* __restrict__ Pin, const double* __restrict__ P0, dou
                     for (int q = 0; q < 5; ++q)
 #pragma unroll
                         for (int m = 0; m < 2 * NG; ++m) S[q][m] = plane[q][TY + m][cx + NG];
-                    hydro_face_flux<Recon, Riem, R>(S, theta, gamma, ny, F);
+                    hydro_face_flux<Recon, Riem, 1, R>(S, theta, gamma, K, ny, F);
 #pragma unroll
                     for (int q = 0; q < 5; ++q) fy[q][TY][cx] = F[q];
                 }
@@ -300,7 +318,7 @@ k_fused_hydro(const double* __restrict__ Pin, const double* __restrict__ P0, dou
 #pragma unroll
             for (int q = 0; q < 5; ++q) p0[q] = P0[q * G.fs + c];
             if constexpr (sizeof(R) == 4) hydro_cons_mixed(igm1, p0, U0);
-            else prim_to_cons<0>(G.gamma, p0, U0);
+            else exact::prim_to_cons<0>(K, p0, U0);
             double Un[5];
 #pragma unroll
             for (int q = 0; q < 5; ++q)
@@ -315,15 +333,22 @@ k_fused_hydro(const double* __restrict__ Pin, const double* __restrict__ P0, dou
             }
             double Pn[5];
             int floor;
+            exact::Recip ir = {1.0, 1.0};
             if constexpr (sizeof(R) == 4) cons_to_prim_mixed<0>(G.gamma, G.pfloor, Un, Pn, floor);
-            else cons_to_prim<0>(G.gamma, G.pfloor, Un, Pn, floor);
+            else exact::cons_to_prim<0>(G.gamma, G.pfloor, Un, Pn, floor, ir);
 #pragma unroll
             for (int q = 0; q < 5; ++q) Pout[q * G.fs + c] = Pn[q];
             if (courant_out)
             {
-                int err = 0;
-                const double d = courant_of<0, R>(Pn, G, err);
-                if (d < dmin) dmin = d;
+                double lmax;
+                if (sizeof(R) == 8 && __builtin_expect(exact::signal_speed<0>(Pn, ir, G.gamma, G.nhat, lmax), 1))
+                    smax = lmax > smax ? lmax : smax;
+                else
+                {
+                    int err = 0;
+                    const double d = courant_of<0, R>(Pn, G, err);
+                    if (d < dmin) dmin = d;
+                }
             }
             if (write_u)
             {
@@ -340,7 +365,15 @@ k_fused_hydro(const double* __restrict__ Pin, const double* __restrict__ P0, dou
         // rewrites after another barrier every wave must reach: the next
         // plane's staging need not wait here (a 2-D tile has one plane)
     }
-    if (courant_out) courant_to_bins(dmin, wmin, TX * TY / 64, tid, ctl);
+    if (courant_out)
+    {
+        if (smax > 0.0)
+        {
+            const double d = G.Lmin / smax;
+            if (d < dmin) dmin = d;
+        }
+        courant_to_bins(dmin, wmin, TX * TY / 64, tid, ctl);
+    }
 }
 
 // The zones of plane k that a TX x TY tile (halo NG = 2) stages from HBM into
@@ -429,20 +462,21 @@ struct PlaneRing
 //   y: h of every row (and the rows above and below the tile) in LDS;
 //   z: h of the zone above computed from the register window and carried.
 // ---------------------------------------------------------------------------
-template <typename R>
-__device__ __forceinline__ R half_slope(R theta, R vl, R v0, R vr)
+// h of five fields; at(q, l, c, r) yields a field's three zones
+template <typename R, typename Zones>
+__device__ __forceinline__ void half_slopes(R theta, Zones at, R* h)
 {
-    return R(+1.0) * R(0.5) * minmod(theta, vl, v0, vr);
-}
-
-template <int Riem, typename R>
-__device__ __forceinline__ void hydro_states_flux(const R* PL, const R* PR, R gamma, const R* n, R* F)
-{
-    State<R, 5> SL, SR;
-    hydro_state(gamma, PL, n, SL);
-    hydro_state(gamma, PR, n, SR);
-    if constexpr (Riem == 1) hllc(SL, SR, n, F);
-    else hlle<R, 5>(SL, SR, F);
+    if constexpr (sizeof(R) == 8) exact::half_slopes<5>(theta, at, h);
+    else
+    {
+#pragma unroll
+        for (int q = 0; q < 5; ++q)
+        {
+            R l, c, r;
+            at(q, l, c, r);
+            h[q] = R(+1.0) * R(0.5) * minmod(theta, l, c, r);
+        }
+    }
 }
 
 // Tile height: binary64 state needs twice the LDS and more VGPRs per lane, so
@@ -476,6 +510,9 @@ __device__ __forceinline__ void fused_plm_tile(const double* __restrict__ Pin, c
     __shared__ double wmin[TX * TY / 64];
 
     double dmin = 1.79769313486231570815e+308;  // this zone column's CFL minimum (last stage)
+    // binary64: the largest signal speed instead; division is monotone, so
+    // the smallest of the quotients Lmin / speed is that of the largest speed
+    double smax = 0.0;
     const int lane = threadIdx.x;
     const int row = threadIdx.y;
     const int tid = row * TX + lane;
@@ -491,6 +528,7 @@ __device__ __forceinline__ void fused_plm_tile(const double* __restrict__ Pin, c
     const long long sxy = (long long)G.N[0] * G.N[1];
     const R theta = R(G.theta), gamma = R(G.gamma);
     const double igm1 = 1.0 / (G.gamma - 1.0);  // binary32 form's U(P0)
+    const exact::Gas K = exact::gas(G.gamma);   // binary64 form
     const R nx[3] = {R(G.nhat[0]), R(G.nhat[1]), R(G.nhat[2])};
     const R ny[3] = {R(G.nhat[3]), R(G.nhat[4]), R(G.nhat[5])};
     const R nz[3] = {R(G.nhat[6]), R(G.nhat[7]), R(G.nhat[8])};
@@ -520,15 +558,16 @@ __device__ __forceinline__ void fused_plm_tile(const double* __restrict__ Pin, c
         }
         // lower z-face of plane kb: zones kb-1 and kb
         R PL[5], PR[5];
+        R hlo[5];
+        half_slopes<R>(theta, [&](int q, R& l, R& c, R& r) { l = w0[q], c = W[q][1], r = W[q][2]; }, hlo);
+        half_slopes<R>(theta, [&](int q, R& l, R& c, R& r) { l = W[q][1], c = W[q][2], r = W[q][3]; }, hzc);
 #pragma unroll
         for (int q = 0; q < 5; ++q)
         {
-            const R hlo = half_slope(theta, w0[q], W[q][1], W[q][2]);
-            hzc[q] = half_slope(theta, W[q][1], W[q][2], W[q][3]);
-            PL[q] = W[q][1] + hlo;
+            PL[q] = W[q][1] + hlo[q];
             PR[q] = W[q][2] + (-hzc[q]);
         }
-        hydro_states_flux<Riem, R>(PL, PR, gamma, nz, Fzlo);
+        hydro_states_flux<Riem, 2, R>(PL, PR, gamma, K, nz, Fzlo);
     }
 
     for (int k = kb; k < ke; ++k)
@@ -563,23 +602,31 @@ __device__ __forceinline__ void fused_plm_tile(const double* __restrict__ Pin, c
                 W[q][1] = W[q][2];
                 W[q][2] = W[q][3];
                 W[q][3] = wn[q];
-                const R hn = half_slope(theta, W[q][1], W[q][2], W[q][3]);
                 PL[q] = W[q][1] + hzc[q];
-                PR[q] = W[q][2] + (-hn);
-                hzc[q] = hn;
             }
-            if (cell_xy) hydro_states_flux<Riem, R>(PL, PR, gamma, nz, Fzhi);
+            half_slopes<R>(theta, [&](int q, R& l, R& c, R& r) { l = W[q][1], c = W[q][2], r = W[q][3]; }, hzc);
+#pragma unroll
+            for (int q = 0; q < 5; ++q) PR[q] = W[q][2] + (-hzc[q]);
+            if (cell_xy) hydro_states_flux<Riem, 2, R>(PL, PR, gamma, K, nz, Fzhi);
         }
         __syncthreads();
 
         // ---- half-slopes: own zone in x (register) and y (LDS); tile-edge zones
-        R hx[5];
+        R hx[5], hy[5];
+        half_slopes<R>(
+            theta,
+            [&](int q, R& l, R& c, R& r) {
+                l = plane[q][row + 2][lane + 1], c = plane[q][row + 2][lane + 2], r = plane[q][row + 2][lane + 3];
+            },
+            hx);
+        half_slopes<R>(
+            theta,
+            [&](int q, R& l, R& c, R& r) {
+                l = plane[q][row + 1][lane + 2], c = plane[q][row + 2][lane + 2], r = plane[q][row + 3][lane + 2];
+            },
+            hy);
 #pragma unroll
-        for (int q = 0; q < 5; ++q)
-        {
-            hx[q] = half_slope(theta, plane[q][row + 2][lane + 1], plane[q][row + 2][lane + 2], plane[q][row + 2][lane + 3]);
-            sy[q][row + 1][lane] = half_slope(theta, plane[q][row + 1][lane + 2], plane[q][row + 2][lane + 2], plane[q][row + 3][lane + 2]);
-        }
+        for (int q = 0; q < 5; ++q) sy[q][row + 1][lane] = hy[q];
         if (lane == TX - 1)
         {
 #pragma unroll
@@ -591,18 +638,30 @@ __device__ __forceinline__ void fused_plm_tile(const double* __restrict__ Pin, c
             {
                 const int cx = tid % TX;
                 const int r = tid < TX ? -1 : TY;
+                R h[5];
+                half_slopes<R>(
+                    theta,
+                    [&](int q, R& lo, R& c, R& up) {
+                        lo = plane[q][r + 1][cx + 2], c = plane[q][r + 2][cx + 2], up = plane[q][r + 3][cx + 2];
+                    },
+                    h);
 #pragma unroll
-                for (int q = 0; q < 5; ++q)
-                    sy[q][r + 1][cx] = half_slope(theta, plane[q][r + 1][cx + 2], plane[q][r + 2][cx + 2], plane[q][r + 3][cx + 2]);
+                for (int q = 0; q < 5; ++q) sy[q][r + 1][cx] = h[q];
             }
             else  // zones i0 - 1 and i0 + 64 of each row
             {
                 const int e = tid - 2 * TX;
                 const int r = e % TY;
                 const int xs = e < TY ? 1 : TX + 2;  // LDS x index of the zone
+                R h[5];
+                half_slopes<R>(
+                    theta,
+                    [&](int q, R& lo, R& c, R& up) {
+                        lo = plane[q][r + 2][xs - 1], c = plane[q][r + 2][xs], up = plane[q][r + 2][xs + 1];
+                    },
+                    h);
 #pragma unroll
-                for (int q = 0; q < 5; ++q)
-                    sxe[q][r][e < TY ? 0 : 2] = half_slope(theta, plane[q][r + 2][xs - 1], plane[q][r + 2][xs], plane[q][r + 2][xs + 1]);
+                for (int q = 0; q < 5; ++q) sxe[q][r][e < TY ? 0 : 2] = h[q];
             }
         }
         __syncthreads();
@@ -625,7 +684,7 @@ __device__ __forceinline__ void fused_plm_tile(const double* __restrict__ Pin, c
                 PL[q] = plane[q][row + 2][lane + 1] + hl[q];
                 PR[q] = plane[q][row + 2][lane + 2] + (-hx[q]);
             }
-            hydro_states_flux<Riem, R>(PL, PR, gamma, nx, Fx);
+            hydro_states_flux<Riem, 0, R>(PL, PR, gamma, K, nx, Fx);
         }
         if (yface)
         {
@@ -636,7 +695,7 @@ __device__ __forceinline__ void fused_plm_tile(const double* __restrict__ Pin, c
                 PL[q] = plane[q][row + 1][lane + 2] + sy[q][row][lane];
                 PR[q] = plane[q][row + 2][lane + 2] + (-sy[q][row + 1][lane]);
             }
-            hydro_states_flux<Riem, R>(PL, PR, gamma, ny, Fy);
+            hydro_states_flux<Riem, 1, R>(PL, PR, gamma, K, ny, Fy);
 #pragma unroll
             for (int q = 0; q < 5; ++q) fy[q][row][lane] = Fy[q];
         }
@@ -656,7 +715,7 @@ __device__ __forceinline__ void fused_plm_tile(const double* __restrict__ Pin, c
                         PL[q] = plane[q][r + 2][TX + 1] + sxe[q][r][1];
                         PR[q] = plane[q][r + 2][TX + 2] + (-sxe[q][r][2]);
                     }
-                    hydro_states_flux<Riem, R>(PL, PR, gamma, nx, F);
+                    hydro_states_flux<Riem, 0, R>(PL, PR, gamma, K, nx, F);
 #pragma unroll
                     for (int q = 0; q < 5; ++q) fxe[q][r] = F[q];
                 }
@@ -672,7 +731,7 @@ __device__ __forceinline__ void fused_plm_tile(const double* __restrict__ Pin, c
                         PL[q] = plane[q][TY + 1][cx + 2] + sy[q][TY][cx];
                         PR[q] = plane[q][TY + 2][cx + 2] + (-sy[q][TY + 1][cx]);
                     }
-                    hydro_states_flux<Riem, R>(PL, PR, gamma, ny, F);
+                    hydro_states_flux<Riem, 1, R>(PL, PR, gamma, K, ny, F);
 #pragma unroll
                     for (int q = 0; q < 5; ++q) fy[q][TY][cx] = F[q];
                 }
@@ -695,7 +754,7 @@ __device__ __forceinline__ void fused_plm_tile(const double* __restrict__ Pin, c
 #pragma unroll
             for (int q = 0; q < 5; ++q) p0[q] = P0[q * G.fs + c];
             if constexpr (sizeof(R) == 4) hydro_cons_mixed(igm1, p0, U0);
-            else prim_to_cons<0>(G.gamma, p0, U0);
+            else exact::prim_to_cons<0>(K, p0, U0);
             double Un[5];
 #pragma unroll
             for (int q = 0; q < 5; ++q)
@@ -710,15 +769,22 @@ __device__ __forceinline__ void fused_plm_tile(const double* __restrict__ Pin, c
             }
             double Pn[5];
             int floor;
+            exact::Recip ir = {1.0, 1.0};
             if constexpr (sizeof(R) == 4) cons_to_prim_mixed<0>(G.gamma, G.pfloor, Un, Pn, floor);
-            else cons_to_prim<0>(G.gamma, G.pfloor, Un, Pn, floor);
+            else exact::cons_to_prim<0>(G.gamma, G.pfloor, Un, Pn, floor, ir);
 #pragma unroll
             for (int q = 0; q < 5; ++q) Pout[q * G.fs + c] = Pn[q];
             if (courant_out)
             {
-                int err = 0;
-                const double d = courant_of<0, R>(Pn, G, err);
-                if (d < dmin) dmin = d;
+                double lmax;
+                if (sizeof(R) == 8 && __builtin_expect(exact::signal_speed<0>(Pn, ir, G.gamma, G.nhat, lmax), 1))
+                    smax = lmax > smax ? lmax : smax;
+                else
+                {
+                    int err = 0;
+                    const double d = courant_of<0, R>(Pn, G, err);
+                    if (d < dmin) dmin = d;
+                }
             }
             if (write_u)
             {
@@ -735,7 +801,15 @@ __device__ __forceinline__ void fused_plm_tile(const double* __restrict__ Pin, c
         // rewrites after another barrier every wave must reach: the next
         // plane's staging need not wait here (a 2-D tile has one plane)
     }
-    if (courant_out) courant_to_bins(dmin, wmin, TX * TY / 64, tid, ctl);
+    if (courant_out)
+    {
+        if (smax > 0.0)
+        {
+            const double d = G.Lmin / smax;
+            if (d < dmin) dmin = d;
+        }
+        courant_to_bins(dmin, wmin, TX * TY / 64, tid, ctl);
+    }
 }
 
 template <int Riem, typename R, bool Z>

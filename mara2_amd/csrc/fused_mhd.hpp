@@ -129,10 +129,10 @@ __device__ __forceinline__ void mhd2d_tile(const double* __restrict__ Pin, const
                 for (int q = 0; q < NQ; ++q)
 #pragma unroll
                     for (int m = 0; m < 2 * NG; ++m) S[q][m] = sP[q][ly][c + m];
-                face_flux<1, Recon, 0, R, A>(S, G, 0, Fq, ctl);
+                face_flux<1, Recon, 0, R, A, 0>(S, G, 0, Fq, ctl);
             }
             else
-                face_flux_at<1, Recon, 0, R, A>(Pin, G, 0, i0 + c, jj, k, Fq, ctl);
+                face_flux_at<1, Recon, 0, R, A, 0>(Pin, G, 0, i0 + c, jj, k, Fq, ctl);
 #pragma unroll
             for (int q = 0; q < NQ; ++q) fx[q][xr_lo + r][c] = Fq[q];
         }
@@ -148,10 +148,10 @@ __device__ __forceinline__ void mhd2d_tile(const double* __restrict__ Pin, const
                 for (int q = 0; q < NQ; ++q)
 #pragma unroll
                     for (int m = 0; m < 2 * NG; ++m) S[q][m] = sP[q][r + m][lx];
-                face_flux<1, Recon, 0, R, A>(S, G, 1, Fq, ctl);
+                face_flux<1, Recon, 0, R, A, 1>(S, G, 1, Fq, ctl);
             }
             else
-                face_flux_at<1, Recon, 0, R, A>(Pin, G, 1, ii, j0 + r, k, Fq, ctl);
+                face_flux_at<1, Recon, 0, R, A, 1>(Pin, G, 1, ii, j0 + r, k, Fq, ctl);
 #pragma unroll
             for (int q = 0; q < NQ; ++q) fy[q][r][yc_lo + c] = Fq[q];
         }
@@ -200,8 +200,11 @@ __device__ __forceinline__ void mhd2d_tile(const double* __restrict__ Pin, const
     if (courant_out) courant_to_bins(dtc, wmin, NT / 64, tid, ctl);
 }
 
+// Binary64 registers are held to what the LDS leaves resident: 3 work-groups
+// of 64 x 4 zones or 2 of 64 x 8 per CU (3 and 4 waves per SIMD).
 template <int Recon, typename R, bool CT, int TY, typename A = Math<R>>
 static __global__ void __launch_bounds__(64 * TY)
+    __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 1 : TY == 4 ? 3 : 4, 8)))
 k_mhd2d(const double* __restrict__ Pin, const double* __restrict__ P0, double* __restrict__ U,
         double* __restrict__ Pout, Geom G, double b, int first_stage, int write_u, int courant_out, Ctl* ctl,
         const double* __restrict__ Ssrc)

@@ -14,6 +14,7 @@
 #pragma once
 
 #include "physics.hpp"
+#include "exact.hpp"
 
 namespace mara {
 
@@ -193,14 +194,27 @@ __device__ __forceinline__ T wave_max(T v)
 // ---------------------------------------------------------------------------
 template <int Recon> struct Stencil { static constexpr int NG = Recon == 0 ? 1 : Recon == 1 ? 2 : 3; };
 
+// Whether (law, precision, arithmetic) is the binary64 form held to the
+// reference's rounding, which exact.hpp evaluates.
+template <int Law, typename R, typename A> struct ReferenceForm
+{
+    static constexpr bool value = sizeof(R) == 8 && Law != 2 && !A::ieee_minmax;
+};
+
 // Flux through one face from the reconstructed primitives on its two sides:
 // the law's face states and the Riemann solver, in arithmetic A (LawMath by
 // default, physics.hpp).
-template <int Law, int Riem, typename R, typename A = LawMath<Law, R>>
+// AX: the axis where the caller knows it at compile time, else -1.
+template <int Law, int Riem, typename R, typename A = LawMath<Law, R>, int AX = -1>
 __device__ __forceinline__ void face_flux_lr(const R* PL, const R* PR, const Geom& G, int axis, R* Fq, Ctl* ctlw)
 {
     constexpr int NQ = LawNQ<Law>::value;
     const R n[3] = {R(G.nhat[3 * axis + 0]), R(G.nhat[3 * axis + 1]), R(G.nhat[3 * axis + 2])};
+    if constexpr (ReferenceForm<Law, R, A>::value)
+    {
+        exact::face_flux<Law, Riem, AX>(PL, PR, exact::gas(G.gamma), n, Fq);
+        return;
+    }
     State<R, NQ> SL, SR;
     const int eL = law_state<Law, R, A>(R(G.gamma), PL, n, SL);
     const int eR = law_state<Law, R, A>(R(G.gamma), PR, n, SR);
@@ -219,7 +233,7 @@ __device__ __forceinline__ void face_flux_lr(const R* PL, const R* PR, const Geo
 
 // Flux through one face from its stencil S[q][m] = P(first stencil zone + m),
 // m = 0 .. 2 NG - 1, in R (reconstruction, law state, Riemann solver).
-template <int Law, int Recon, int Riem, typename R, typename A = LawMath<Law, R>>
+template <int Law, int Recon, int Riem, typename R, typename A = LawMath<Law, R>, int AX = -1>
 __device__ __forceinline__ void face_flux(const R (&S)[LawNQ<Law>::value][2 * Stencil<Recon>::NG], const Geom& G,
                                           int axis, R* Fq, Ctl* ctlw)
 {
@@ -227,6 +241,22 @@ __device__ __forceinline__ void face_flux(const R (&S)[LawNQ<Law>::value][2 * St
     constexpr int NG = Stencil<Recon>::NG;
     R PL[NQ], PR[NQ];
     const R theta = R(G.theta);
+    if constexpr (NG == 2 && ReferenceForm<Law, R, A>::value)
+    {
+        double hl[NQ], hr[NQ];
+        exact::half_slopes<NQ>(
+            theta, [&](int q, double& l, double& c, double& r) { l = S[q][0], c = S[q][1], r = S[q][2]; }, hl);
+        exact::half_slopes<NQ>(
+            theta, [&](int q, double& l, double& c, double& r) { l = S[q][1], c = S[q][2], r = S[q][3]; }, hr);
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+        {
+            PL[q] = S[q][1] + hl[q];
+            PR[q] = S[q][2] - hr[q];
+        }
+        face_flux_lr<Law, Riem, R, A, AX>(PL, PR, G, axis, Fq, ctlw);
+        return;
+    }
 #pragma unroll
     for (int q = 0; q < NQ; ++q)
     {
@@ -246,12 +276,12 @@ __device__ __forceinline__ void face_flux(const R (&S)[LawNQ<Law>::value][2 * St
             PR[q] = weno5<R, false, A>(S[q][1], S[q][2], S[q][3], S[q][4], S[q][5]);
         }
     }
-    face_flux_lr<Law, Riem, R, A>(PL, PR, G, axis, Fq, ctlw);
+    face_flux_lr<Law, Riem, R, A, AX>(PL, PR, G, axis, Fq, ctlw);
 }
 
 // Flux through the face left of cell (i, j, k) along axis, from the stencil
 // of 2 NG cells read from P.
-template <int Law, int Recon, int Riem, typename R, typename A = LawMath<Law, R>>
+template <int Law, int Recon, int Riem, typename R, typename A = LawMath<Law, R>, int AX = -1>
 __device__ __forceinline__ void face_flux_at(const double* __restrict__ P, const Geom& G, int axis, int i, int j,
                                              int k, R* Fq, Ctl* ctlw)
 {
@@ -278,7 +308,7 @@ __device__ __forceinline__ void face_flux_at(const double* __restrict__ P, const
             PR[q] = weno5<R, false, A>(v[1], v[2], v[3], v[4], v[5]);
             asm volatile("" : : "v"(PL[q]), "v"(PR[q]) : "memory");
         }
-        face_flux_lr<Law, Riem, R, A>(PL, PR, G, axis, Fq, ctlw);
+        face_flux_lr<Law, Riem, R, A, AX>(PL, PR, G, axis, Fq, ctlw);
         return;
     }
     R S[NQ][2 * NG];
@@ -289,16 +319,16 @@ __device__ __forceinline__ void face_flux_at(const double* __restrict__ P, const
 #pragma unroll
         for (int m = 0; m < 2 * NG; ++m) S[q][m] = R(Pq[m * stride]);
     }
-    face_flux<Law, Recon, Riem, R, A>(S, G, axis, Fq, ctlw);
+    face_flux<Law, Recon, Riem, R, A, AX>(S, G, axis, Fq, ctlw);
 }
 
-template <int Law, int Recon, int Riem, typename R>
+template <int Law, int Recon, int Riem, typename R, int AX>
 __device__ __forceinline__ void flux_face(const double* __restrict__ P, R* __restrict__ F, const Geom& G, int axis,
                                           int i, int j, int k, Ctl* ctlw)
 {
     constexpr int NQ = LawNQ<Law>::value;
     R Fq[NQ];
-    face_flux_at<Law, Recon, Riem, R>(P, G, axis, i, j, k, Fq, ctlw);
+    face_flux_at<Law, Recon, Riem, R, LawMath<Law, R>, AX>(P, G, axis, i, j, k, Fq, ctlw);
     const long long f = face_index(G, i, j, k);
 #pragma unroll
     for (int q = 0; q < NQ; ++q) F[q * G.ffs + f] = Fq[q];
@@ -307,9 +337,11 @@ __device__ __forceinline__ void flux_face(const double* __restrict__ P, R* __res
 // Threads over the (m0, m1, m2) face box: 64 x rows work-groups with z from
 // the grid, or (linear != 0) a 1-D grid over the box's faces in x-fastest
 // order, which keeps every lane busy where m0 is not a multiple of 64 (the
-// flux-CT ring makes it 2 more than the interior).
-template <int Law, int Recon, int Riem, typename R>
-static __global__ void __launch_bounds__(256)
+// flux-CT ring makes it 2 more than the interior).  The bit-exact binary64
+// form compiles one kernel per axis (AX): its faces use that the axis normals
+// hold exact zeros and ones.
+template <int Law, int Recon, int Riem, typename R, int AX>
+static __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AX < 0 ? 1 : 4, 8)))
 k_flux(const double* __restrict__ P, R* __restrict__ F, const Geom G, int axis,
        int lo0, int lo1, int lo2, int m0, int m1, int m2, int linear, Ctl* ctl)
 {
@@ -331,7 +363,7 @@ k_flux(const double* __restrict__ P, R* __restrict__ F, const Geom G, int axis,
         tk = (int)blockIdx.z;
         if (ti >= m0 || tj >= m1) return;
     }
-    flux_face<Law, Recon, Riem, R>(P, F, G, axis, lo0 + ti, lo1 + tj, lo2 + tk, ctl);
+    flux_face<Law, Recon, Riem, R, AX>(P, F, G, AX < 0 ? axis : AX, lo0 + ti, lo1 + tj, lo2 + tk, ctl);
 }
 
 // ---------------------------------------------------------------------------
@@ -579,7 +611,9 @@ __device__ __forceinline__ double finish_zone(const double* __restrict__ P0, dou
     double p0[NQ], U0[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) p0[q] = P0[q * G.fs + c];
-    if (prim_to_cons<Law>(G.gamma, p0, U0) != ERR_NONE) atomicAdd(&ctl->superluminal, 1ull);
+    constexpr bool EXACT = ReferenceForm<Law, R, A>::value;
+    if constexpr (EXACT) exact::prim_to_cons<Law>(exact::gas(G.gamma), p0, U0);
+    else if (prim_to_cons<Law>(G.gamma, p0, U0) != ERR_NONE) atomicAdd(&ctl->superluminal, 1ull);
 
     double Un[NQ];
 #pragma unroll
@@ -595,7 +629,9 @@ __device__ __forceinline__ double finish_zone(const double* __restrict__ P0, dou
     double Pn[NQ];
     int floor = 0;
     int failed;
-    if constexpr (MIX || FAST) failed = cons_to_prim_mixed<Law>(G.gamma, G.pfloor, Un, Pn, floor);
+    exact::Recip ir = {1.0, 1.0};  // of the zone's new density (EXACT)
+    if constexpr (EXACT) failed = exact::cons_to_prim<Law>(G.gamma, G.pfloor, Un, Pn, floor, ir);
+    else if constexpr (MIX || FAST) failed = cons_to_prim_mixed<Law>(G.gamma, G.pfloor, Un, Pn, floor);
     else failed = cons_to_prim<Law>(G.gamma, G.pfloor, Un, Pn, floor);
     if (failed != 0)
     {
@@ -617,7 +653,10 @@ __device__ __forceinline__ double finish_zone(const double* __restrict__ P0, dou
             // as FieldOperator::getCourantTimestep reads them)
             int err = 0;
             const double Lz = zone_length(G, i, j, k);
+            double lmax;
             if constexpr (MIX) dtc = courant_of<Law, float>(Pn, G, Lz, err);
+            else if (EXACT && __builtin_expect(exact::signal_speed<EXACT ? Law : 0>(Pn, ir, G.gamma, G.nhat, lmax), 1))
+                dtc = Lz / lmax;
             else dtc = courant_of<Law, double, A>(Pn, G, Lz, err);
             if (err & ERR_SUPERLUMINAL) atomicAdd(&ctl->superluminal, 1ull);
             if (err & ERR_EIGEN) atomicAdd(&ctl->eigen_fail, 1ull);
@@ -801,7 +840,7 @@ __device__ __forceinline__ double pencil_tile(const double* __restrict__ Pin, co
             for (int m = 0; m < 2 * NG; ++m) S[q][m] = sP[q * W + t + m];
         }
         R Fq[NQ];
-        face_flux<Law, Recon, Riem, R>(S, G, 0, Fq, ctl);
+        face_flux<Law, Recon, Riem, R, LawMath<Law, R>, 0>(S, G, 0, Fq, ctl);
 #pragma unroll
         for (int q = 0; q < NQ; ++q) sF[q * PENCIL + t] = Fq[q];
     }

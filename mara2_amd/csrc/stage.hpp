@@ -59,6 +59,23 @@ constexpr int ROWS_SHAPES[3] = {1, 2, 4};
 inline dim3 stage_block3(int rows) { return dim3(64, rows, 1); }
 inline dim3 stage_grid3(int m0, int m1, int m2, int rows) { return dim3((m0 + 63) / 64, (m1 + rows - 1) / rows, m2); }
 
+template <int Law, int Recon, int Riem, typename R, int AX>
+void flux_sweep(const StageArgs& s, int axis, const int* lo, const int* hi)
+{
+    const Geom& G = *s.G;
+    const int m0 = hi[0] - lo[0], m1 = hi[1] - lo[1], m2 = hi[2] - lo[2];
+    // rows of 64 lanes leave (64 - m0 % 64) lanes of each row's last
+    // wavefront idle; past an eighth of the lanes the faces go in one line
+    const int padded = (m0 + 63) / 64 * 64;
+    const long long faces = (long long)m0 * m1 * m2;
+    if (8 * (padded - m0) > padded && faces < (1ll << 31))
+        k_flux<Law, Recon, Riem, R, AX><<<(unsigned)((faces + 255) / 256), 256, 0, s.stream>>>(
+            s.Pin, (R*)s.F[axis], G, axis, lo[0], lo[1], lo[2], m0, m1, m2, 1, s.ctl);
+    else
+        k_flux<Law, Recon, Riem, R, AX><<<stage_grid3(m0, m1, m2, s.rows), stage_block3(s.rows), 0, s.stream>>>(
+            s.Pin, (R*)s.F[axis], G, axis, lo[0], lo[1], lo[2], m0, m1, m2, 0, s.ctl);
+}
+
 template <int Law, int Recon, int Riem, typename R>
 void stage_flux_t(const StageArgs& s, int axis)
 {
@@ -75,17 +92,14 @@ void stage_flux_t(const StageArgs& s, int axis)
             hi[a] = G.N[a] - G.g[a] + ring;
         }
     }
-    const int m0 = hi[0] - lo[0], m1 = hi[1] - lo[1], m2 = hi[2] - lo[2];
-    // rows of 64 lanes leave (64 - m0 % 64) lanes of each row's last
-    // wavefront idle; past an eighth of the lanes the faces go in one line
-    const int padded = (m0 + 63) / 64 * 64;
-    const long long faces = (long long)m0 * m1 * m2;
-    if (8 * (padded - m0) > padded && faces < (1ll << 31))
-        k_flux<Law, Recon, Riem, R><<<(unsigned)((faces + 255) / 256), 256, 0, s.stream>>>(
-            s.Pin, (R*)s.F[axis], G, axis, lo[0], lo[1], lo[2], m0, m1, m2, 1, s.ctl);
+    if constexpr (ReferenceForm<Law, R, LawMath<Law, R>>::value)
+    {
+        if (axis == 0) flux_sweep<Law, Recon, Riem, R, 0>(s, axis, lo, hi);
+        else if (axis == 1) flux_sweep<Law, Recon, Riem, R, 1>(s, axis, lo, hi);
+        else flux_sweep<Law, Recon, Riem, R, 2>(s, axis, lo, hi);
+    }
     else
-        k_flux<Law, Recon, Riem, R><<<stage_grid3(m0, m1, m2, s.rows), stage_block3(s.rows), 0, s.stream>>>(
-            s.Pin, (R*)s.F[axis], G, axis, lo[0], lo[1], lo[2], m0, m1, m2, 0, s.ctl);
+        flux_sweep<Law, Recon, Riem, R, -1>(s, axis, lo, hi);
 }
 
 template <int Law, typename R>
