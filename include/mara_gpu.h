@@ -258,7 +258,9 @@ typedef struct mara_shape
 
 /* The block's launch shape.  A new block starts from the tuning table's
    entry for its descriptor, else from pencil 256, zplanes 16 and rows 4
-   (rows 2 for a fused 2-D MHD block).
+   (rows 2 for a fused 2-D MHD block); until a shape is set or tuned, a fused
+   3-D block's stages march the planes that suit its size and the device
+   rather than 16.
    set: MARA_ERR_INVALID_ARGUMENT for a value outside the lists above. */
 int mara_block_get_shape(const mara_block* block, mara_shape* shape);
 int mara_block_set_shape(mara_block* block, const mara_shape* shape);

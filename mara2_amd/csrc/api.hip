@@ -98,6 +98,7 @@ struct mara_block
     int pencil = 0;  // 1-D pencil tile length (pencil_supported), else 0
     bool mhd2d = false;  // fused 2-D MHD tiles (mhd2d_supported)
     int kz = FUSED_KZ;           // fused 3-D kernels: z planes per work-group
+    int kz_rule = 0;             // the planes taken while no shape was set or tuned (fused_planes), else 0
     int rows = ROWS_DEFAULT;     // flux-array kernels: work-group rows
     int pencil_shape = PENCIL_DEFAULT;  // requested pencil length (all laws)
     bool in_group = false;    // a group member: the group's exchange fills its guards
@@ -317,7 +318,7 @@ void launch_stage(mara_block* b, int rk, int courant_out)
     s.ct = b->S.ct;
     s.pencil = b->pencil;
     s.mhd2d = b->mhd2d;
-    s.kz = b->kz;
+    s.kz = b->kz_rule ? b->kz_rule : b->kz;
     s.rows = b->rows;
     s.S = b->src_fn || cooling ? b->Ssrc : nullptr;
     s.wrap = wrap;
@@ -395,6 +396,7 @@ void apply_shape(mara_block* b, const mara_shape& s)
     b->pencil_shape = s.pencil;
     if (b->pencil) b->pencil = pencil_length(b->d.law, s.pencil);
     b->kz = s.zplanes;
+    b->kz_rule = 0;
     b->rows = s.rows;
     // the captured steps hold the old launch shape
     if (b->steps_exec) (void)hipGraphExecDestroy(b->steps_exec);
@@ -439,6 +441,33 @@ int capture_steps(mara_block* b)
         return MARA_ERR_HIP;
     }
     return MARA_OK;
+}
+
+// Work-groups of the block's fused 3-D kernel resident per CU, its tiles per z
+// layer and the device's CUs (zeros where they cannot be had).
+void fused_round(const mara_block* b, int* per_cu, int* per_layer, int* cus)
+{
+    StageArgs q;
+    q.d = &b->d;
+    q.G = &b->G;
+    q.fused = b->fused;
+    int dev = 0;
+    *per_cu = *per_layer = 0;
+    stage_round(q, b->d.precision == MARA_PREC_MIXED, per_cu, per_layer);
+    if (hipGetDevice(&dev) != hipSuccess
+        || hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        *cus = 0;
+    (void)hipGetLastError();
+}
+
+// The planes per work-group of a fused 3-D block without a shape of its own;
+// blocks: how many like it run side by side (a group's members).
+void choose_planes(mara_block* b, int blocks)
+{
+    if (!b->fused || b->G.N[2] < 2) return;
+    int per_cu = 0, per_layer = 0, cus = 0;
+    fused_round(b, &per_cu, &per_layer, &cus);
+    b->kz_rule = fused_planes((long long)per_layer * blocks, b->G.n[2], per_cu, cus);
 }
 
 int read_ctl(mara_block* b)
@@ -510,6 +539,7 @@ int mara_block_create(const mara_desc* d, mara_block** out)
     {
         mara_shape tuned;
         if (tune_find(*d, &tuned)) apply_shape(b, tuned);
+        else choose_planes(b, 1);
     }
 
     auto fail = [&](int code) { mara_block_destroy(b); return code; };
@@ -618,15 +648,8 @@ int mara_block_autotune(mara_block* b, int repeats, mara_shape* chosen, double* 
         // rounds, each round every CU holding as many work-groups as the
         // kernel's occupancy allows: no partly filled last round, and fewer
         // tiles re-reading the z window at their start
-        StageArgs q;
-        q.d = &b->d;
-        q.G = &b->G;
-        int per_cu = 0, per_layer = 0, cus = 0, dev = 0;
-        stage_round(q, b->d.precision == MARA_PREC_MIXED, &per_cu, &per_layer);
-        if (hipGetDevice(&dev) != hipSuccess
-            || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-            cus = 0;
-        (void)hipGetLastError();
+        int per_cu = 0, per_layer = 0, cus = 0;
+        fused_round(b, &per_cu, &per_layer, &cus);
         for (int r = 1; r <= 3 && per_cu > 0 && per_layer > 0 && cus > 0; ++r)
         {
             const long long layers = (long long)r * per_cu * cus / per_layer;
@@ -1251,6 +1274,7 @@ extern "C" int mara_advance_noalloc(const mara_desc* d, const double* P_in, doub
     b.mhd2d = mhd2d_supported(d);
     if (b.mhd2d) b.rows = MHD_ROWS_DEFAULT;
     b.G = make_geom(*d);
+    choose_planes(&b, 1);
     const ScratchPlan plan = plan_scratch(*d, b.S, b.fused || b.pencil || b.mhd2d);
     if (plan.total > MARA_SCRATCH_BYTES) return MARA_ERR_CAPACITY;
     int dev = -1;
@@ -1533,6 +1557,7 @@ int mara_group_create(const mara_desc* d, const int* dims, mara_group** out)
         mara_block* b = g->blocks[m];
         b->in_group = true;
         b->graphs = false;
+        if (b->kz_rule) choose_planes(b, g->count);
         for (int a = 0; a < 3; ++a) b->G.dA[a] = whole.dA[a];
         b->G.dV = whole.dV;
         b->G.Lmin = whole.Lmin;

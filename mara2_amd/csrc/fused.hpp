@@ -914,6 +914,46 @@ inline void fused_round_t(const Geom& G, int* per_cu, int* per_layer)
     *per_cu = n;
 }
 
+// z planes per work-group of a block whose shape nobody set: the count with
+// the shortest stage by a model of the tiles' march.  A tile of k planes costs
+// k + 1/2 (its prologue reads three planes and solves a face), 1 + 0.4 (n - 1)
+// times as much where n work-groups share its CU.  The tiles run in rounds of
+// per_cu per CU, the last round on fewer per CU; as neighbours drift apart the
+// rounds blend into an even spread, so the two are averaged 3 : 2.  Few planes
+// give a small block enough tiles to fill the chip (one wavefront per SIMD
+// marches at its own latency, whatever the others do), and counts whose last
+// round is nearly empty are passed over.  The search ends at 32: beyond, the
+// marches drift so far apart that neighbours no longer find each other's halo
+// planes in L2 (fast 256^3: 16 planes 652 us, 86 planes, one exact round, 671);
+// and the default stays where the model promises under 3 %.  Measured, stage
+// in us, 16 planes -> the rule's (its pick within 2 % of the best of 2 .. 128
+// planes for eight boxes from 32^3 to 256^3 in each form): bit-exact 64^3 131
+// -> 35 (2), 96 x 80 x 200 214 -> 160 (4), 161 x 142 x 118 355 -> 266 (17);
+// fast 64^3 66 -> 21, 128^3 98 -> 90; mixed 64^3 75 -> 19, 192^3 265 -> 243.
+inline int fused_planes(long long per_layer, int n2, int per_cu, int cus)
+{
+    if (per_layer < 1 || per_cu < 1 || cus < 1 || n2 < 1) return FUSED_KZ;
+    const auto shared = [](double n) { return 1.0 + 0.4 * (n - 1.0); };
+    const long long slots = (long long)per_cu * cus;
+    int best = FUSED_KZ;
+    double least = 1e300, at_default = 1e300;
+    for (int k = 2; k <= 32 && (k == 2 || k <= n2); ++k)
+    {
+        const long long tiles = per_layer * ((n2 + k - 1) / k), full = tiles / slots, rest = tiles % slots;
+        double t = full * shared(per_cu);
+        if (rest) t += shared((double)((rest + cus - 1) / cus));
+        if (full) t = 0.6 * t + 0.4 * (double)tiles / slots * shared(per_cu);
+        t *= k + 0.5;
+        if (t < least)
+        {
+            least = t;
+            best = k;
+        }
+        if (k == FUSED_KZ) at_default = t;
+    }
+    return least > 0.97 * at_default ? FUSED_KZ : best;
+}
+
 template <typename R>
 inline void fused_round_r(const mara_desc& d, const Geom& G, int* per_cu, int* per_layer)
 {
