@@ -222,8 +222,9 @@ int mara_block_set_viscous_flux(mara_block* block, const char* code_object, cons
 
 /* mara_block_run replays its steps from a HIP graph of 16 steps, captured on
    the first run (enable=1, the default), or launches every kernel from the
-   host (enable=0).  Results are the same either way; runs with stage timing
-   enabled launch from the host.  No counterpart in the reference: the
+   host (enable=0); 1-D hydro and MHD blocks in RK2 without hooks take many
+   steps per launch instead of a graph.  Results are the same either way; runs
+   with stage timing enabled launch from the host.  No counterpart in the reference: the
    reference steps on the host. */
 int mara_block_set_graphs(mara_block* block, int enable);
 

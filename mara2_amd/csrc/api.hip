@@ -26,6 +26,7 @@
 #include "fused.hpp"
 #include "host_common.hpp"
 #include "stage.hpp"
+#include "run1d.hpp"
 
 using namespace mara;
 using namespace mara::host;
@@ -470,6 +471,34 @@ void choose_planes(mara_block* b, int blocks)
     b->kz_rule = fused_planes((long long)per_layer * blocks, b->G.n[2], per_cu, cus);
 }
 
+// Whether the block's steps run on chip (run1d.hpp): 1-D hydro and MHD in RK2
+// without hooks, while stages are not timed one by one.  Fills the launch's
+// arguments but for the step counts.
+bool run1d_args(mara_block* b, run1d::Args* a)
+{
+    if (!b->pencil || b->src_fn || b->vis_fn || b->timing || b->in_group || !run1d::supported(b->d)) return false;
+    a->d = &b->d;
+    a->G = &b->G;
+    a->stream = b->stream;
+    a->Pa = b->Pa;
+    a->Pb = b->Pb;
+    a->ctl = b->ctl;
+    a->host = b->ctl_host;
+    a->box = reinterpret_cast<unsigned long long*>(b->U);  // the RK state, which these steps keep in registers
+    a->decision = reinterpret_cast<unsigned*>(&b->ctl->pad);
+    a->threads = run1d::one_threads(b->d, b->ng);
+    a->groups = a->threads ? 1 : run1d::split_groups(b->d, b->ng);
+    a->max_steps = 1;
+    a->given = 0;
+    a->dt = 0.0;
+    return a->threads || (a->groups && a->groups * run1d::group_bytes(b->d, b->ng) <= (long long)b->S.nq * b->S.fs * 8);
+}
+
+void run1d_launch(mara_block* b, const run1d::Args& a)
+{
+    b->d.precision == MARA_PREC_MIXED ? run1d::launch_f32(a) : run1d::launch_f64(a);
+}
+
 int read_ctl(mara_block* b)
 {
     HIP_TRY(hipMemcpyAsync(b->ctl_host, b->ctl, sizeof(Ctl), hipMemcpyDeviceToHost, b->stream));
@@ -852,6 +881,17 @@ int mara_block_advance(mara_block* b, double t0, double dt, mara_report* report)
 {
     (void)t0;
     if (!b) return MARA_ERR_INVALID_ARGUMENT;
+    run1d::Args a;
+    if (run1d_args(b, &a) && a.threads)
+    {
+        // a 1-D block of one work-group: the step and its report in one launch
+        a.given = 1;
+        a.dt = dt;
+        run1d_launch(b, a);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipStreamSynchronize(b->stream));
+        return fill_report(b, report);
+    }
     k_ctl_begin_advance<<<1, 1, 0, b->stream>>>(b->ctl, dt);
     for (int rk = 0; rk < b->d.rk_order; ++rk) launch_stage(b, rk, 0);
     HIP_TRY(hipGetLastError());
@@ -863,12 +903,22 @@ int mara_block_advance(mara_block* b, double t0, double dt, mara_report* report)
 int mara_block_courant_dt(mara_block* b, double* dt)
 {
     if (!b || !dt) return MARA_ERR_INVALID_ARGUMENT;
-    k_ctl_begin_courant<<<1, 1, 0, b->stream>>>(b->ctl);
-    launch_courant(b);
-    k_ctl_fold_bins<<<1, 1, 0, b->stream>>>(b->ctl);
-    HIP_TRY(hipGetLastError());
-    int e = read_ctl(b);
-    if (e) return e;
+    run1d::Args a;
+    if (run1d_args(b, &a) && a.threads)
+    {
+        b->d.precision == MARA_PREC_MIXED ? run1d::courant_f32(a) : run1d::courant_f64(a);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipStreamSynchronize(b->stream));
+    }
+    else
+    {
+        k_ctl_begin_courant<<<1, 1, 0, b->stream>>>(b->ctl);
+        launch_courant(b);
+        k_ctl_fold_bins<<<1, 1, 0, b->stream>>>(b->ctl);
+        HIP_TRY(hipGetLastError());
+        const int e = read_ctl(b);
+        if (e) return e;
+    }
     union { unsigned long long u; double d; } cv;
     cv.u = b->ctl_host->courant_bits;
     *dt = cv.d;
@@ -900,9 +950,12 @@ int mara_block_run(mara_block* b, double cfl, double t_final, int max_steps,
     // stage timing records events around each stage launch, which a graph
     // replay would overwrite: timed runs launch eagerly
     const bool graph = b->graphs && !b->timing;
-    if (graph && !b->steps_exec)
+    run1d::Args chip;
+    bool on_chip = graph && run1d_args(b, &chip);
+    const auto capture = [&]() { return graph && !b->steps_exec ? capture_steps(b) : MARA_OK; };
+    if (!on_chip)
     {
-        const int e = capture_steps(b);
+        const int e = capture();
         if (e) return e;
     }
     k_ctl_begin_run<<<1, 1, 0, b->stream>>>(b->ctl, *t, t_final, cfl, max_steps);
@@ -910,6 +963,45 @@ int mara_block_run(mara_block* b, double cfl, double t_final, int max_steps,
     launch_courant(b);
     constexpr int kChunk = 64;
     int queued = 0, chunk = kChunk;
+    bool current = false;  // whether ctl_host holds the control block as the device left it
+    if (on_chip)
+    {
+        // a split block reads its neighbours' zones in place of the guards of
+        // a periodic mesh: the first step, whose guards the caller may have
+        // filled otherwise, goes by launches
+        if (!chip.threads)
+        {
+            queued = max_steps < 1 ? max_steps : 1;
+            enqueue_steps(b, queued);
+        }
+        // steps per launch: bounds the time the GPU is held without a break
+        constexpr int kOnChip = 16384;
+        while (queued < max_steps)
+        {
+            chip.max_steps = max_steps - queued < kOnChip ? max_steps - queued : kOnChip;
+            run1d_launch(b, chip);
+            queued += chip.max_steps;
+            HIP_TRY(hipGetLastError());
+            const int e = read_ctl(b);
+            if (e) return e;
+            current = true;
+            const Ctl& c = *b->ctl_host;
+            if (!chip.threads && c.pad == (int)run1d::GAVE_UP)
+            {
+                // the work-groups were not resident together: by launches
+                on_chip = false;
+                queued = c.steps;
+                break;
+            }
+            if (!c.active || !(c.t < c.t_final) || c.steps >= max_steps || ctl_status(c) != MARA_OK) break;
+        }
+        if (on_chip) queued = max_steps;
+        else
+        {
+            const int e = capture();
+            if (e) return e;
+        }
+    }
     while (queued < max_steps)
     {
         // enqueue a chunk of steps; steps after the stop condition are no-ops
@@ -921,8 +1013,9 @@ int mara_block_run(mara_block* b, double cfl, double t_final, int max_steps,
         enqueue_steps(b, chunk - s);
         queued += chunk;
         HIP_TRY(hipGetLastError());
-        int e = read_ctl(b);
+        const int e = read_ctl(b);
         if (e) return e;
+        current = true;
         const Ctl& c = *b->ctl_host;
         if (!c.active || !(c.t < c.t_final) || c.steps >= max_steps) break;
         // size the next chunk to the steps the clock still needs at the last
@@ -931,8 +1024,11 @@ int mara_block_run(mara_block* b, double cfl, double t_final, int max_steps,
         chunk = kChunk;
         if (c.dt > 0 && left + 8 < kChunk) chunk = (int)left + 8;
     }
-    int e = read_ctl(b);
-    if (e) return e;
+    if (!current)
+    {
+        const int e = read_ctl(b);
+        if (e) return e;
+    }
     *t = b->ctl_host->t;
     *steps = b->ctl_host->steps;
     return fill_report(b, report);

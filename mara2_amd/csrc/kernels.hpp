@@ -597,6 +597,58 @@ __device__ __forceinline__ void write_guard_images(double* __restrict__ P, const
 // A: the arithmetic of the zone's CFL wave speeds (LawMath; Rel in the fast
 // binary64 form, which also recovers the primitives with one reciprocal of
 // the density, as the mixed form does).
+// What a stage makes of one zone.
+template <int Law> struct ZoneResult
+{
+    double U[LawNQ<Law>::value], P[LawNQ<Law>::value];  // P is not set where the recovery failed
+    int failed, floor;                                  // recovery failure, floor used
+    exact::Recip ir;                                    // of the new density (binary64 of the reference's rounding)
+};
+
+// The update itself: U0 from the step's starting primitives p0, the RK
+// combine with the stage's conserved state uq(q) (U0 in a first stage) and
+// the flux divergence lq(q), and the primitives.  False where p0 is
+// superluminal.
+template <int Law, typename R, typename A, typename Uof, typename Lof>
+__device__ __forceinline__ bool zone_update(const Geom& G, double dt, double b, int first_stage, const double* p0,
+                                            Uof uq, Lof lq, ZoneResult<Law>& z)
+{
+    constexpr int NQ = LawNQ<Law>::value;
+    constexpr bool EXACT = ReferenceForm<Law, R, A>::value;
+    constexpr bool MIX = sizeof(R) == 4 && Law < 2;
+    constexpr bool FAST = sizeof(R) == 8 && Law < 2 && A::ieee_minmax;
+    bool fine = true;
+    double U0[NQ];
+    if constexpr (EXACT) exact::prim_to_cons<Law>(exact::gas(G.gamma), p0, U0);
+    else fine = prim_to_cons<Law>(G.gamma, p0, U0) == ERR_NONE;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+    {
+        const double Uq = first_stage ? U0[q] : uq(q);
+        const double Lq = lq(q);
+        z.U[q] = U0[q] * (1 - b) + (Uq + dt * Lq) * b;
+    }
+    z.floor = 0;
+    z.ir = {1.0, 1.0};
+    if constexpr (EXACT) z.failed = exact::cons_to_prim<Law>(G.gamma, G.pfloor, z.U, z.P, z.floor, z.ir);
+    else if constexpr (MIX || FAST) z.failed = cons_to_prim_mixed<Law>(G.gamma, G.pfloor, z.U, z.P, z.floor);
+    else z.failed = cons_to_prim<Law>(G.gamma, G.pfloor, z.U, z.P, z.floor);
+    return fine;
+}
+
+// The CFL time step of the updated zone on a cell length Lz.
+template <int Law, typename R, typename A>
+__device__ __forceinline__ double zone_cfl(const Geom& G, double Lz, const ZoneResult<Law>& z, int& err)
+{
+    constexpr bool EXACT = ReferenceForm<Law, R, A>::value;
+    constexpr bool MIX = sizeof(R) == 4 && Law < 2;
+    if constexpr (MIX) return courant_of<Law, float>(z.P, G, Lz, err);
+    double lmax;
+    if (EXACT && __builtin_expect(exact::signal_speed<EXACT ? Law : 0>(z.P, z.ir, G.gamma, G.nhat, lmax), 1))
+        return Lz / lmax;
+    return courant_of<Law, double, A>(z.P, G, Lz, err);
+}
+
 template <int Law, typename R = double, typename A = LawMath<Law, R>>
 __device__ __forceinline__ double finish_zone(const double* __restrict__ P0, double* __restrict__ U,
                                               double* __restrict__ Pout, const Geom& G, double b, int first_stage,
@@ -608,65 +660,44 @@ __device__ __forceinline__ double finish_zone(const double* __restrict__ P0, dou
     const long long c = cell_index(G, i, j, k);
     const double dt = ctl->dt;
 
-    double p0[NQ], U0[NQ];
+    double p0[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) p0[q] = P0[q * G.fs + c];
-    constexpr bool EXACT = ReferenceForm<Law, R, A>::value;
-    if constexpr (EXACT) exact::prim_to_cons<Law>(exact::gas(G.gamma), p0, U0);
-    else if (prim_to_cons<Law>(G.gamma, p0, U0) != ERR_NONE) atomicAdd(&ctl->superluminal, 1ull);
-
-    double Un[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; ++q)
-    {
-        const double Uq = first_stage ? U0[q] : U[q * G.fs + c];
+    ZoneResult<Law> z;
+    const bool fine = zone_update<Law, R, A>(
+        G, dt, b, first_stage, p0, [&](int q) { return U[q * G.fs + c]; },
         // L += S (src/SolutionSchemes.cpp:209-217) when a source is set
-        const double Lq = Ssrc ? L[q] + Ssrc[q * G.fs + c] : L[q];
-        Un[q] = U0[q] * (1 - b) + (Uq + dt * Lq) * b;
-    }
-    constexpr bool MIX = sizeof(R) == 4 && Law < 2;
-    constexpr bool FAST = sizeof(R) == 8 && Law < 2 && A::ieee_minmax;
-    double Pn[NQ];
-    int floor = 0;
-    int failed;
-    exact::Recip ir = {1.0, 1.0};  // of the zone's new density (EXACT)
-    if constexpr (EXACT) failed = exact::cons_to_prim<Law>(G.gamma, G.pfloor, Un, Pn, floor, ir);
-    else if constexpr (MIX || FAST) failed = cons_to_prim_mixed<Law>(G.gamma, G.pfloor, Un, Pn, floor);
-    else failed = cons_to_prim<Law>(G.gamma, G.pfloor, Un, Pn, floor);
-    if (failed != 0)
+        [&](int q) { return Ssrc ? L[q] + Ssrc[q * G.fs + c] : L[q]; }, z);
+    if (!fine) atomicAdd(&ctl->superluminal, 1ull);
+    if (z.failed != 0)
     {
         atomicAdd(&ctl->c2p_fail, 1ull);
         atomicMin(&ctl->first_fail, ref_linear(G, i, j, k));
         // the zone keeps its previous value, and so do its ghost images
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) Pn[q] = Pout[q * G.fs + c];
-        write_guard_images<NQ>(Pout, G, i, j, k, Pn);
+        for (int q = 0; q < NQ; ++q) z.P[q] = Pout[q * G.fs + c];
+        write_guard_images<NQ>(Pout, G, i, j, k, z.P);
     }
     else
     {
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) Pout[q * G.fs + c] = Pn[q];
-        write_guard_images<NQ>(Pout, G, i, j, k, Pn);
+        for (int q = 0; q < NQ; ++q) Pout[q * G.fs + c] = z.P[q];
+        write_guard_images<NQ>(Pout, G, i, j, k, z.P);
         if (courant_out)
         {
             // the next step's CFL from the zone's new primitives (interior only,
             // as FieldOperator::getCourantTimestep reads them)
             int err = 0;
-            const double Lz = zone_length(G, i, j, k);
-            double lmax;
-            if constexpr (MIX) dtc = courant_of<Law, float>(Pn, G, Lz, err);
-            else if (EXACT && __builtin_expect(exact::signal_speed<EXACT ? Law : 0>(Pn, ir, G.gamma, G.nhat, lmax), 1))
-                dtc = Lz / lmax;
-            else dtc = courant_of<Law, double, A>(Pn, G, Lz, err);
+            dtc = zone_cfl<Law, R, A>(G, zone_length(G, i, j, k), z, err);
             if (err & ERR_SUPERLUMINAL) atomicAdd(&ctl->superluminal, 1ull);
             if (err & ERR_EIGEN) atomicAdd(&ctl->eigen_fail, 1ull);
         }
     }
-    if (floor) atomicAdd(&ctl->floor_applied, 1ull);
+    if (z.floor) atomicAdd(&ctl->floor_applied, 1ull);
     if (write_u)
     {
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) U[q * G.fs + c] = Un[q];
+        for (int q = 0; q < NQ; ++q) U[q * G.fs + c] = z.U[q];
     }
     return dtc;
 }
