@@ -27,6 +27,7 @@
 #include "host_common.hpp"
 #include "stage.hpp"
 #include "run1d.hpp"
+#include "transfer.hpp"
 
 using namespace mara;
 using namespace mara::host;
@@ -102,6 +103,7 @@ struct mara_block
     int kz_rule = 0;             // the planes taken while no shape was set or tuned (fused_planes), else 0
     int rows = ROWS_DEFAULT;     // flux-array kernels: work-group rows
     int pencil_shape = PENCIL_DEFAULT;  // requested pencil length (all laws)
+    bool pool_user = false;   // counted by lane_pool (transfer.hpp)
     bool in_group = false;    // a group member: the group's exchange fills its guards
     // the guards of Pa may not hold the ghost fill of its interior: the
     // stages of the PLM tiles of a periodic block neither read nor fill them
@@ -617,6 +619,8 @@ int mara_block_create(const mara_desc* d, mara_block** out)
     if (!hip_ok(hipMemset(b->Pa, 0, cellbytes))) return fail(MARA_ERR_HIP);
     if (!hip_ok(hipMemset(b->Pb, 0, cellbytes))) return fail(MARA_ERR_HIP);
     b->bytes = device_bytes(d, b->S);
+    b->pool_user = true;
+    lane_pool().add_user();
     *out = b;
     return MARA_OK;
 }
@@ -642,6 +646,7 @@ int mara_block_destroy(mara_block* b)
     for (int e = 0; e < 2 * mara_block::kTimingPairs; ++e)
         if (b->ev[e]) hipEventDestroy(b->ev[e]);
     if (b->stream) hipStreamDestroy(b->stream);
+    if (b->pool_user) lane_pool().drop_user();
     delete b;
     return MARA_OK;
 }
@@ -845,8 +850,14 @@ int mara_tune_load(const char* path)
 int mara_block_upload_prim(mara_block* b, const double* P)
 {
     if (!b || !P) return MARA_ERR_INVALID_ARGUMENT;
-    const size_t n = (size_t)b->S.ncell * b->S.nq;
-    HIP_TRY(hipMemcpyAsync(b->U, P, n * sizeof(double), hipMemcpyHostToDevice, b->stream));
+    const size_t bytes = (size_t)b->S.ncell * b->S.nq * sizeof(double);
+    if (bytes >= THRESHOLD)
+    {
+        HIP_TRY(hipStreamSynchronize(b->stream));
+        HIP_TRY(copy_large(reinterpret_cast<char*>(b->U), reinterpret_cast<char*>(const_cast<double*>(P)), bytes, true));
+    }
+    else
+        HIP_TRY(hipMemcpyAsync(b->U, P, bytes, hipMemcpyHostToDevice, b->stream));
     k_aos_to_soa<<<grid_for(b->S.ncell), kThreads, 0, b->stream>>>(b->U, b->Pa, b->G);
     b->guards_stale = false;
     HIP_TRY(hipGetLastError());
@@ -857,11 +868,17 @@ int mara_block_upload_prim(mara_block* b, const double* P)
 int mara_block_download_prim(mara_block* b, double* P)
 {
     if (!b || !P) return MARA_ERR_INVALID_ARGUMENT;
-    const size_t n = (size_t)b->S.ncell * b->S.nq;
+    const size_t bytes = (size_t)b->S.ncell * b->S.nq * sizeof(double);
     fill_guards(b);
     k_soa_to_aos<<<grid_for(b->S.ncell), kThreads, 0, b->stream>>>(b->Pa, b->U, b->G);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(P, b->U, n * sizeof(double), hipMemcpyDeviceToHost, b->stream));
+    if (bytes >= THRESHOLD)
+    {
+        HIP_TRY(hipStreamSynchronize(b->stream));
+        HIP_TRY(copy_large(reinterpret_cast<char*>(b->U), reinterpret_cast<char*>(P), bytes, false));
+        return MARA_OK;
+    }
+    HIP_TRY(hipMemcpyAsync(P, b->U, bytes, hipMemcpyDeviceToHost, b->stream));
     HIP_TRY(hipStreamSynchronize(b->stream));
     return MARA_OK;
 }
