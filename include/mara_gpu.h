@@ -362,7 +362,9 @@ int mara_batch_step(mara_batch* batch, int n_steps, int* n_active);
 /* With enable=1 (the default) mara_batch_step launches one round of kernels
    (a step of the large solves and the small 1-D solves' steps beside it) as a
    HIP graph, captured when the set of solves changed and replayed n_steps
-   times; with enable=0 it launches every kernel from the host.  Results are
+   times, and 1-D hydro and MHD solves of an RK2 batch take their steps of the
+   call in one launch beside it; with enable=0 it launches every kernel from
+   the host.  Results are
    the same either way.  No counterpart in the reference. */
 int mara_batch_set_graphs(mara_batch* batch, int enable);
 

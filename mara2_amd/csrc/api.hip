@@ -488,12 +488,12 @@ bool run1d_args(mara_block* b, run1d::Args* a)
     a->host = b->ctl_host;
     a->box = reinterpret_cast<unsigned long long*>(b->U);  // the RK state, which these steps keep in registers
     a->decision = reinterpret_cast<unsigned*>(&b->ctl->pad);
-    a->threads = run1d::one_threads(b->d, b->ng);
-    a->groups = a->threads ? 1 : run1d::split_groups(b->d, b->ng);
+    a->threads = run1d::one_threads(b->G.n[0], b->ng);
+    a->groups = a->threads ? 1 : run1d::split_groups(b->G.n[0], b->ng, b->G.nq, b->G.fs);
     a->max_steps = 1;
     a->given = 0;
     a->dt = 0.0;
-    return a->threads || (a->groups && a->groups * run1d::group_bytes(b->d, b->ng) <= (long long)b->S.nq * b->S.fs * 8);
+    return a->groups > 0;
 }
 
 void run1d_launch(mara_block* b, const run1d::Args& a)
@@ -983,16 +983,9 @@ int mara_block_run(mara_block* b, double cfl, double t_final, int max_steps,
     bool current = false;  // whether ctl_host holds the control block as the device left it
     if (on_chip)
     {
-        // a split block reads its neighbours' zones in place of the guards of
-        // a periodic mesh: the first step, whose guards the caller may have
-        // filled otherwise, goes by launches
-        if (!chip.threads)
-        {
-            queued = max_steps < 1 ? max_steps : 1;
-            enqueue_steps(b, queued);
-        }
         // steps per launch: bounds the time the GPU is held without a break
         constexpr int kOnChip = 16384;
+        bool tried = false;
         while (queued < max_steps)
         {
             chip.max_steps = max_steps - queued < kOnChip ? max_steps - queued : kOnChip;
@@ -1005,9 +998,19 @@ int mara_block_run(mara_block* b, double cfl, double t_final, int max_steps,
             const Ctl& c = *b->ctl_host;
             if (!chip.threads && c.pad == (int)run1d::GAVE_UP)
             {
+                queued = c.steps;
+                if (queued == 0 && !tried)
+                {
+                    // guards that are not the boundary condition's images:
+                    // the first step by launches, which leave images
+                    tried = true;
+                    enqueue_steps(b, 1);
+                    queued = 1;
+                    current = false;
+                    continue;
+                }
                 // the work-groups were not resident together: by launches
                 on_chip = false;
-                queued = c.steps;
                 break;
             }
             if (!c.active || !(c.t < c.t_final) || c.steps >= max_steps || ctl_status(c) != MARA_OK) break;

@@ -79,6 +79,15 @@ void box_tiles(std::vector<BTile>& out, int item, const int lo[3], const int hi[
     }
 }
 
+// Work-groups a pencil-class solve runs on on chip (run1d.hpp): 0 where it
+// goes by launches (the relativistic law, solves too long for it, one that gave
+// up before, and with graphs off every solve).
+int chip_parts(const mara_batch* B, const Slot& sl, const Geom& G, int ng)
+{
+    if (!B->graphs || sl.by_launches || sl.d.law == MARA_LAW_RMHD) return 0;
+    return run1d::split_groups(G.n[0], ng, G.nq, G.fs);
+}
+
 void build_table(mara_batch* B)
 {
     B->table_version += 1;
@@ -86,6 +95,8 @@ void build_table(mara_batch* B)
     for (int a = 0; a < 3; ++a) B->flux[a].clear();
     B->update.clear();
     B->ghost.clear();
+    B->chips.clear();
+    B->chip_segments.clear();
     auto seg_begin = [&]() { return (int)B->tiles.size(); };
     for (size_t c = 0; c < B->classes.size(); ++c)
     {
@@ -141,13 +152,30 @@ void build_table(mara_batch* B)
         }
         if (B->classes[c].pencil)
         {
-            // one tile per pl - 1 interior zones of each 1-D item
+            // solves that run on chip, in launches of CHIP_RESIDENT work-groups
+            int o = (int)B->chips.size();
+            const auto close = [&]() {
+                const int count = (int)B->chips.size() - o;
+                if (count > 0) B->chip_segments.push_back(ChipSegment{(int)c, o, count});
+                o = (int)B->chips.size();
+            };
+            for (int n = 0; n < B->n_items; ++n)
+            {
+                const Slot& sl = B->slots[n];
+                if (!sl.used || sl.cls != (int)c) continue;
+                const int parts = chip_parts(B, sl, B->items[n].G, recon_ng(B->classes[c].recon));
+                B->items[n].lane = parts ? LANE_CHIP : B->classes[c].lane;
+                if ((int)B->chips.size() - o + parts > CHIP_RESIDENT) close();
+                for (int w = 0; w < parts; ++w) B->chips.push_back(BChip{n, w, parts, 0});
+            }
+            close();
+            // one tile per pl - 1 interior zones of each other 1-D item
             const int pl = pencil_length(B->classes[c].law, B->pencil);
             const int s0 = seg_begin();
             for (int n = 0; n < B->n_items; ++n)
             {
                 const Slot& sl = B->slots[n];
-                if (!sl.used || sl.cls != (int)c) continue;
+                if (!sl.used || sl.cls != (int)c || B->items[n].lane == LANE_CHIP) continue;
                 const Geom& G = B->items[n].G;
                 const int ie = G.N[0] - G.g[0];
                 for (int x0 = G.g[0]; x0 < ie; x0 += pl - 1)
@@ -207,6 +235,15 @@ int upload_table(mara_batch* B)
     }
     if (!B->tiles.empty())
         HIP_TRY(hipMemcpyAsync(B->d_tiles, B->tiles.data(), B->tiles.size() * sizeof(BTile), hipMemcpyHostToDevice, B->stream));
+    if ((int)B->chips.size() > B->chip_capacity)
+    {
+        if (B->d_chips) HIP_TRY(hipFree(B->d_chips));
+        B->d_chips = nullptr;
+        B->chip_capacity = (int)std::max<size_t>(B->chips.size() * 2, 256);
+        HIP_TRY(hipMalloc(&B->d_chips, B->chip_capacity * sizeof(BChip)));
+    }
+    if (!B->chips.empty())
+        HIP_TRY(hipMemcpyAsync(B->d_chips, B->chips.data(), B->chips.size() * sizeof(BChip), hipMemcpyHostToDevice, B->stream));
     if (B->n_items)
         HIP_TRY(hipMemcpyAsync(B->d_items, B->items.data(), B->n_items * sizeof(BItem), hipMemcpyHostToDevice, B->stream));
     return MARA_OK;
@@ -362,6 +399,7 @@ int mara_batch_destroy(mara_batch* B)
     (void)hipFree(B->d_ctl);
     (void)hipFree(B->d_bins);
     (void)hipFree(B->d_tiles);
+    (void)hipFree(B->d_chips);
     (void)hipFree(B->d_queue);
     (void)hipFree(B->d_src[0]);
     (void)hipFree(B->d_src[1]);
@@ -465,7 +503,7 @@ int mara_batch_set_express(mara_batch* B, int max_solves)
 int mara_batch_lane(const mara_batch* B, int slot, int* lane)
 {
     if (!B || !lane || slot < 0 || slot >= B->max_solves || !B->slots[slot].used) return MARA_ERR_INVALID_ARGUMENT;
-    *lane = B->items[slot].lane;
+    *lane = B->items[slot].lane == LANE_CHIP ? 1 : B->items[slot].lane;
     return MARA_OK;
 }
 
@@ -492,6 +530,7 @@ int mara_batch_set_shape(mara_batch* B, const mara_shape* shape)
 int mara_batch_set_graphs(mara_batch* B, int enable)
 {
     if (!B) return MARA_ERR_INVALID_ARGUMENT;
+    if (B->graphs != (enable != 0)) B->dirty = true;  // solves on chip and by launches change places
     B->graphs = enable != 0;
     return MARA_OK;
 }
@@ -560,6 +599,7 @@ int mara_batch_admit(mara_batch* B, const mara_desc* d, const double* P, double 
         else it.cfl = key.law < 2 ? fast64::CFL_MIXED : fast64::CFL_EXACT;
     }
     sl.express = false;
+    sl.by_launches = false;
 
     Ctl& c = B->h_ctl[n];
     std::memset(&c, 0, sizeof c);
@@ -649,15 +689,16 @@ int mara_batch_step(mara_batch* B, int n_steps, int* n_active)
     }
     const int n = B->n_items;
     const unsigned ig = (unsigned)((n + 63) / 64);
-    // Three lanes: tile kernels (2-D/3-D solves, and 1-D ones outside RK2) on
-    // the first stream, pencil kernels of 1-D RK2 solves on the second, so
+    // Lanes: tile kernels (2-D/3-D solves, and 1-D ones outside RK2) on the
+    // first stream, 1-D RK2 solves on the second (on chip, several hundred
+    // steps per launch, or by pencil kernels where that is not to be had), so
     // that small 1-D solves are not held to the pace of large ones, and the
     // express lane (promote_long_chains) on the third.  A round is one
     // tile-lane step; the other lanes take `ratio` / `ratio3` steps in it,
     // sized from the tile lane's estimated step time (its active zones at
     // ~5e9 zone-stages per second, plus ~20 us of launches) against theirs.
-    long long zones[3] = {0, 0, 0};
-    bool busy[3] = {false, false, false};
+    long long zones[4] = {0, 0, 0, 0};
+    bool busy[4] = {false, false, false, false};
     for (int k = 0; k < n; ++k)
     {
         if (!B->slots[k].used || finished(B->h_ctl[k])) continue;
@@ -671,6 +712,17 @@ int mara_batch_step(mara_batch* B, int n_steps, int* n_active)
     int ratio = 1, ratio3 = 1;
     if (any_pencil && (any_tile || any_express)) ratio = (int)std::min(32.0, std::max(1.0, round_time / 20e-6));
     if (any_express && any_tile) ratio3 = (int)std::min(32.0, std::max(1.0, round_time / step_time(2)));
+    // the solves on chip take as many steps as fit a round beside the tile
+    // lane, at ~7 us a step for each of the launches that follow one another:
+    // hydro on the second stream, MHD on the third
+    int chip_steps = 0;
+    if (busy[LANE_CHIP])
+    {
+        int launches[2] = {0, 0};
+        for (const ChipSegment& s : B->chip_segments) ++launches[B->classes[s.cls].law != MARA_LAW_HYDRO];
+        const double fit = any_tile || any_express ? round_time / (7e-6 * std::max(launches[0], launches[1])) : 1.0;
+        chip_steps = n_steps * (int)std::min(32.0, std::max(1.0, fit));
+    }
     const unsigned sg = (unsigned)((n + 3) / 4);  // kb_step_start: 4 items per work-group
     // `count` steps of one lane: one kernel ends a step and starts the next
     auto run_lane = [&](int lane, int count) {
@@ -687,7 +739,7 @@ int mara_batch_step(mara_batch* B, int n_steps, int* n_active)
         }
     };
     auto run_round = [&]() {
-        if (any_tile || (!any_pencil && !any_express))
+        if (any_tile || (!any_pencil && !any_express && !chip_steps))
         {
             B->cur = B->stream;
             run_lane(0, 1);
@@ -704,7 +756,30 @@ int mara_batch_step(mara_batch* B, int n_steps, int* n_active)
         }
     };
     const int lanes = (any_tile ? 1 : 0) | (any_pencil ? 2 : 0) | (any_express ? 4 : 0);
-    if (B->graphs && n > 0 && n_steps > 1)
+    // beside the rounds, from where the first stream stands
+    const auto launch_chips = [&]() {
+        HIP_TRY(hipEventRecord(B->fork, B->stream));
+        HIP_TRY(hipStreamWaitEvent(B->stream2, B->fork, 0));
+        HIP_TRY(hipStreamWaitEvent(B->stream3, B->fork, 0));
+        for (const ChipSegment& s : B->chip_segments)
+        {
+            const hipStream_t to = B->classes[s.cls].law == MARA_LAW_HYDRO ? B->stream2 : B->stream3;
+            B->precision == MARA_PREC_MIXED ? run_chip_f32(B, s, chip_steps, to) : run_chip<double>(B, s, chip_steps, to);
+        }
+        HIP_TRY(hipEventRecord(B->join, B->stream2));
+        HIP_TRY(hipEventRecord(B->join3, B->stream3));
+        return (int)MARA_OK;
+    };
+    const auto join_chips = [&]() {
+        HIP_TRY(hipStreamWaitEvent(B->stream, B->join, 0));
+        HIP_TRY(hipStreamWaitEvent(B->stream, B->join3, 0));
+        return (int)MARA_OK;
+    };
+    if (chip_steps && !lanes)
+    {
+        if (launch_chips() || join_chips()) return MARA_ERR_HIP;
+    }
+    else if (B->graphs && n > 0 && n_steps > 1)
     {
         if (!B->round_exec || B->round_version != B->table_version || B->round_n != n || B->round_ratio != ratio
             || B->round_ratio3 != ratio3 || B->round_lanes != lanes)
@@ -743,13 +818,16 @@ int mara_batch_step(mara_batch* B, int n_steps, int* n_active)
             B->round_ratio3 = ratio3;
             B->round_lanes = lanes;
         }
+        if (chip_steps && launch_chips()) return MARA_ERR_HIP;
         for (int s = 0; s < n_steps; ++s) HIP_TRY(hipGraphLaunch(B->round_exec, B->stream));
+        if (chip_steps && join_chips()) return MARA_ERR_HIP;
     }
     else
     {
         HIP_TRY(hipEventRecord(B->fork, B->stream));
         HIP_TRY(hipStreamWaitEvent(B->stream2, B->fork, 0));
         HIP_TRY(hipStreamWaitEvent(B->stream3, B->fork, 0));
+        if (chip_steps && launch_chips()) return MARA_ERR_HIP;
         for (int s = 0; s < n_steps && n > 0; ++s) run_round();
         HIP_TRY(hipEventRecord(B->join, B->stream2));
         HIP_TRY(hipEventRecord(B->join3, B->stream3));
@@ -766,6 +844,13 @@ int mara_batch_step(mara_batch* B, int n_steps, int* n_active)
         const Ctl& c = B->h_ctl[k];
         if (!B->slots[k].used) continue;
         if (!finished(c)) ++active;
+        // work-groups that were not resident together, or guards that are not
+        // the boundary condition's: nothing happened; pencil kernels from here
+        if (B->items[k].lane == LANE_CHIP && c.pad == (int)run1d::GAVE_UP)
+        {
+            B->slots[k].by_launches = true;
+            B->dirty = true;
+        }
     }
     if (n_active) *n_active = active;
     return MARA_OK;

@@ -16,6 +16,7 @@
 #include "fused.hpp"
 #include "fused_mhd.hpp"
 #include "fused_fast.hpp"
+#include "run1d.hpp"
 
 namespace mara {
 
@@ -28,7 +29,8 @@ struct BItem
     void* F[3];
     Ctl* ctl;
     int bc;
-    int lane;  // 0: tile kernels on the batch's first stream, 1: pencil kernels on the second
+    int lane;  // 0: tile kernels on the batch's first stream, 1: pencil kernels on the second,
+               // 2: express, 3: on chip (run1d.hpp)
     int cfl;   // arithmetic of the CFL time step of the item's stage kernels (fast64::CflArith)
     double* S; // NewtonianMHD cooling terms of the stage (nine-field items), else null
 };
@@ -120,6 +122,39 @@ kb_pencil(const BItem* __restrict__ items, const BTile* __restrict__ tiles, doub
     const double dtc = pencil_tile<Law, Recon, Riem, R, CT, PENCIL>(Pin, it.Pa, it.U, Pout, it.G, b, first, !last,
                                                                     courant_out, it.ctl, T.x0, sP, sF, nullptr);
     if (courant_out) courant_to_bins(dtc, wmin, PENCIL / 64, threadIdx.x, it.ctl);
+}
+
+// 1-D items of an RK2 batch on chip: up to max_steps of their steps in one
+// launch.  A table entry names a work-group's item and its part of it; the
+// item's RK state holds the messages of its work-groups and its control block
+// their decision, as for a single block (run1d.hpp).
+struct BChip
+{
+    int item;
+    int part, parts;
+    int pad;
+};
+
+static __global__ void __launch_bounds__(256)
+kb_run1d_open(const BItem* __restrict__ items, const BChip* __restrict__ chips, int words)
+{
+    const BChip C = chips[blockIdx.x];
+    const BItem& it = items[C.item];
+    unsigned long long* box = reinterpret_cast<unsigned long long*>(it.U) + (long long)C.part * words;
+    for (int t = threadIdx.x; t < words; t += 256) box[t] = run1d::EMPTY;
+    if (C.part == 0 && threadIdx.x == 0) it.ctl->pad = run1d::OPEN;
+}
+
+template <int Law, int Recon, int Riem, typename R, bool CT>
+static __global__ void __launch_bounds__(run1d::PL)
+kb_run1d(const BItem* __restrict__ items, const BChip* __restrict__ chips, int max_steps)
+{
+    const BChip C = chips[blockIdx.x];
+    const BItem& it = items[C.item];
+    const Geom G = it.G;
+    run1d::run<Law, Recon, Riem, R, CT, run1d::PL, false>(
+        it.Pa, it.Pb, G, it.ctl, C.part, C.parts, max_steps, 0, 0.0, reinterpret_cast<unsigned long long*>(it.U),
+        reinterpret_cast<unsigned*>(&it.ctl->pad), run1d::PATIENCE, nullptr);
 }
 
 // 2-D and 3-D hydro + PLM items of an RK2 batch: the single block's fused

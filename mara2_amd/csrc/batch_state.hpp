@@ -74,6 +74,7 @@ struct Slot
     bool used = false;
     bool fresh = false;
     bool express = false;  // a long chain moved to the express lane
+    bool by_launches = false;  // a 1-D solve whose run on chip gave up: pencil kernels from then on
     mara_desc d;
     int cls = -1;
     long long off = 0, bytes = 0;
@@ -95,6 +96,19 @@ struct ClassKey
 };
 
 struct Segment { int offset, count; };
+
+// Work-groups of solves that run on chip (run1d.hpp): one launch each.
+struct ChipSegment
+{
+    int cls;
+    int offset, count;
+};
+// The work-groups of a solve must be resident together, beside tile kernels:
+// at most this many of 256 threads per launch, with two launches side by side
+// (hydro and MHD) under two work-groups per CU
+constexpr int CHIP_RESIDENT = 224;
+// lane of the solves that run on chip (mara_batch_lane reports the pencil lane, 1)
+constexpr int LANE_CHIP = 3;
 
 } // namespace batch
 } // namespace mara
@@ -147,6 +161,10 @@ struct mara_batch
     std::map<int, mara::batch::Segment> flux[3];  // class -> segment
     std::map<int, mara::batch::Segment> update;
     std::map<int, mara::batch::Segment> ghost;     // fused classes: ghost-zone tiles
+    std::vector<mara::BChip> chips;                // work-groups of the solves on chip
+    std::vector<mara::batch::ChipSegment> chip_segments;
+    mara::BChip* d_chips = nullptr;
+    int chip_capacity = 0;
     long long table_version = 0;                   // bumped by every table build
     // HIP graph of one round (a tile-lane step and `ratio` pencil-lane steps),
     // replayed n_steps times by mara_batch_step; recaptured when the table,
@@ -338,8 +356,28 @@ void run_stage(mara_batch* B, int rk, int lane)
 }
 
 
+// `steps` steps at most of one segment of solves on chip, on `stream`
+template <int Law, int Recon, int Riem, typename R, bool CT>
+void chip_launch(mara_batch* B, const ChipSegment& s, int steps, hipStream_t stream)
+{
+    const BChip* t = B->d_chips + s.offset;
+    kb_run1d_open<<<s.count, 256, 0, stream>>>(B->d_items, t, run1d::SLOTS * run1d::Message<Law, Recon>::WORDS);
+    kb_run1d<Law, Recon, Riem, R, CT><<<s.count, run1d::PL, 0, stream>>>(B->d_items, t, steps);
+}
+
+template <typename R>
+void run_chip(mara_batch* B, const ChipSegment& s, int steps, hipStream_t stream)
+{
+    const ClassKey& k = B->classes[s.cls];
+#define CH(L, Rc, Rm, C) if (k.law == L && k.recon == Rc && k.riemann == Rm && k.ct == C) { chip_launch<L, Rc, Rm, R, (C != 0)>(B, s, steps, stream); return; }
+    CH(0, 0, 0, 0) CH(0, 0, 1, 0) CH(0, 1, 0, 0) CH(0, 1, 1, 0) CH(0, 2, 0, 0) CH(0, 2, 1, 0)
+    CH(1, 0, 0, 0) CH(1, 1, 0, 0) CH(1, 2, 0, 0) CH(1, 0, 0, 1) CH(1, 1, 0, 1) CH(1, 2, 0, 1)
+#undef CH
+}
+
 // binary32 stage launches, compiled with contraction in mixed.hip
 void run_stage_f32(mara_batch* B, int rk, int lane);
+void run_chip_f32(mara_batch* B, const ChipSegment& s, int steps, hipStream_t stream);
 
 } // namespace batch
 } // namespace mara

@@ -16,6 +16,10 @@ void stage_round_f32(const StageArgs& s, int* per_cu, int* per_layer) { fused_ro
 
 namespace batch {
 void run_stage_f32(mara_batch* B, int rk, int lane) { run_stage<float>(B, rk, lane); }
+void run_chip_f32(mara_batch* B, const ChipSegment& s, int steps, hipStream_t stream)
+{
+    run_chip<float>(B, s, steps, stream);
+}
 } // namespace batch
 
 } // namespace mara

@@ -1,5 +1,7 @@
 // run1d.hpp -- many RK2 steps of a 1-D block in one launch (mara_block_run,
-// mara_block_advance).
+// mara_block_advance), and of the 1-D solves of a batch (mara_batch_step,
+// kb_run1d: the serving mix of 48 solves, 240 steps each, 60 -> 50 ms, the 1-D
+// solves' share no longer the longest).
 //
 // A 1-D step is small: at 1024 zones its two stage kernels and the step
 // boundary were 14 us of launches and memory latency around 1 us of
@@ -128,11 +130,12 @@ __device__ __forceinline__ void report(const Ctl* ctl, Ctl* host, int m)
 // k_ctl_begin_advance starts it, with the control block's copy left in host
 // memory.  ONE: a block of one work-group of THREADS threads; only such a
 // block takes given steps.
+// w of groups: this work-group's part.
 template <int Law, int Recon, int Riem, typename R, bool CT, int THREADS, bool ONE>
-static __global__ void __launch_bounds__(THREADS)
-k_run1d(double* __restrict__ Pa, double* __restrict__ Pb, const Geom G, Ctl* __restrict__ ctl, int max_steps,
-        int given, double dt_given, unsigned long long* __restrict__ box, unsigned* __restrict__ decision,
-        int patience, Ctl* __restrict__ host)
+__device__ __forceinline__ void run(double* __restrict__ Pa, double* __restrict__ Pb, const Geom& G,
+                                    Ctl* __restrict__ ctl, int w, int groups, int max_steps, int given,
+                                    double dt_given, unsigned long long* __restrict__ box,
+                                    unsigned* __restrict__ decision, int patience, Ctl* __restrict__ host)
 {
     constexpr int NQ = LawNQ<Law>::value, NG = Stencil<Recon>::NG;
     constexpr int LO = ONE ? NG : 2 * NG;  // local index of the first own zone
@@ -147,7 +150,6 @@ k_run1d(double* __restrict__ Pa, double* __restrict__ Pb, const Geom G, Ctl* __r
 
     const int m = threadIdx.x, lane = m & 63, wave = m >> 6;
     const int n = G.n[0], g = G.g[0];
-    const int groups = gridDim.x, w = blockIdx.x;
     // own zones [r0, r0 + nz) of the interior, spread evenly
     const int q0 = n / groups, extra = n % groups;
     const int nz = q0 + (w < extra ? 1 : 0), r0 = w * q0 + (w < extra ? w : extra);
@@ -196,6 +198,15 @@ k_run1d(double* __restrict__ Pa, double* __restrict__ Pb, const Geom G, Ctl* __r
     {
 #pragma unroll
         for (int q = 0; q < NQ; ++q) sP[q][m] = R(P[q]);
+        if (wraps && ((r < 0 && r >= -NG) || (r >= n && r < n + NG)))
+        {
+            // guards that are not the periodic images (as uploaded) count in
+            // the first step, which then goes by launches
+            bool image = true;
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) image = image && dbits(Pa[q * G.fs + g + r]) == dbits(P[q]);
+            if (!image) atomicCAS(decision, (unsigned)OPEN, (unsigned)GAVE_UP);
+        }
     }
     if (m == 0) lost = 0;
     __syncthreads();
@@ -489,6 +500,16 @@ k_run1d(double* __restrict__ Pa, double* __restrict__ Pb, const Geom G, Ctl* __r
     }
 }
 
+template <int Law, int Recon, int Riem, typename R, bool CT, int THREADS, bool ONE>
+static __global__ void __launch_bounds__(THREADS)
+k_run1d(double* __restrict__ Pa, double* __restrict__ Pb, const Geom G, Ctl* __restrict__ ctl, int max_steps,
+        int given, double dt_given, unsigned long long* __restrict__ box, unsigned* __restrict__ decision,
+        int patience, Ctl* __restrict__ host)
+{
+    run<Law, Recon, Riem, R, CT, THREADS, ONE>(Pa, Pb, G, ctl, (int)blockIdx.x, (int)gridDim.x, max_steps, given,
+                                               dt_given, box, decision, patience, host);
+}
+
 // The CFL time step of a block of one work-group, in one launch: k_courant
 // (or the mixed form's k_courant_form) between k_ctl_begin_courant and
 // k_ctl_fold_bins, the control block's copy left in host memory.
@@ -533,25 +554,20 @@ k_courant_one(const double* __restrict__ P, const Geom G, Ctl* __restrict__ ctl,
 // wavefronts per SIMD and no exchange, is level with three of 256 (508 zones,
 // hydro 5.7 us a step against 6.3, MHD 10.2 against 9.8); above that the
 // split is faster.
-inline int one_threads(const mara_desc& d, int ng)
+inline int one_threads(int cells, int ng)
 {
-    const int need = d.cells[0] + 2 * ng;
+    const int need = cells + 2 * ng;
     return need <= 256 ? 256 : need <= 512 ? 512 : 0;
 }
 
-inline int split_groups(const mara_desc& d, int ng)
+// fs: the field stride of the block's RK state, which holds the messages
+inline int split_groups(int cells, int ng, int nq, long long fs)
 {
     const int most = PL - 4 * ng;  // own zones of a work-group
-    const int groups = (d.cells[0] + most - 1) / most;
+    const int groups = (cells + most - 1) / most;
+    const long long words = (long long)SLOTS * (1 + 2 * 2 * ng * nq);  // of one work-group
     // every work-group holds at least the zones its neighbours' halos take
-    return groups <= GROUPS_MAX && d.cells[0] / groups >= 2 * ng ? groups : 0;
-}
-
-// message bytes of one work-group
-inline long long group_bytes(const mara_desc& d, int ng)
-{
-    const int nq = d.law == MARA_LAW_HYDRO ? 5 : 8;
-    return (long long)SLOTS * (1 + 2 * 2 * ng * nq) * 8;
+    return groups <= GROUPS_MAX && cells / groups >= 2 * ng && groups * words <= nq * fs ? groups : 0;
 }
 
 struct Args

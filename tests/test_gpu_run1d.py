@@ -112,3 +112,37 @@ def test_host_loop_equals_oracle(n, law):
             err, _ = oracle.advance(desc, Po, 0.0, 0.4 * dt)
             assert err == 0
         assert np.array_equal(blk.download(), Po)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_solves_of_a_batch(precision):
+    """1-D solves of every kind and length together on chip, some in more
+    work-groups than one launch holds, one with guards that are not its
+    boundary condition's (it goes by launches), against the batch that launches
+    every kernel from the host: the same states, clocks, steps and statuses,
+    whatever the steps per call."""
+    from mara2_amd.runtime import Batch
+    kinds = []
+    for k, n in enumerate([3, 60, 248, 249, 252, 700, 1000, 3001, 16384, 16384, 16384, 16384, 49000, 51000]):
+        law = "mhd" if k % 2 else "hydro"
+        bc = ("outflow", "periodic", "reflecting")[k % 3]
+        recon = ("plm", "plm", "weno5", "pcm")[k % 4]
+        desc = abi.make_desc(law=law, recon=recon, bc=bc, cells=(n, 1, 1), precision=precision, pressure_floor=1e-6,
+                             riemann="hllc" if law == "hydro" else "hlle")
+        kinds.append((desc, _random(desc, seed=k, guards=k != 4), 1e300 if k % 2 else 0.3 / n, 40 + k))
+    assert kinds[4][0].bc == abi.BC_PERIODIC
+    seen = []
+    for graphs, chunk in ((False, 16), (True, 16), (True, 1)):
+        with Batch(1 << 29, precision=precision, max_solves=len(kinds)) as b:
+            b.set_graphs(graphs)
+            slots = [b.admit(d, P, 0.4, t, s) for d, P, t, s in kinds]
+            assert None not in slots and all(b.lane(s) == 1 for s in slots)
+            calls = 0
+            while b.step(chunk):
+                calls += 1
+                assert calls < 200
+            state = [b.query(s) for s in slots]
+            seen.append(([(q[0], q[1], q[2], q[3], q[4].as_dict()) for q in state], [b.retire(s) for s in slots]))
+    for info, states in seen[1:]:
+        assert info == seen[0][0]
+        assert all(np.array_equal(a, c) for a, c in zip(states, seen[0][1]))
