@@ -22,6 +22,15 @@ using namespace mara::batch;
 
 namespace {
 
+void drop_graphs(mara_batch* B)
+{
+    for (LaneGraph& g : B->lane_graph)
+    {
+        if (g.exec) (void)hipGraphExecDestroy(g.exec);
+        g.exec = nullptr;
+    }
+}
+
 int class_of(mara_batch* B, const mara_desc& d, bool express = false)
 {
     const bool one_d = d.cells[1] == 1 && d.cells[2] == 1;
@@ -38,7 +47,7 @@ int class_of(mara_batch* B, const mara_desc& d, bool express = false)
     else if (plain && !one_d && rk2 && law == MARA_LAW_MHD && d.cells[2] == 1) fused = 3;
     const int pencil = (plain && one_d && rk2 && law != LAW_MHD_COOLING) ? 1 : 0;
     const ClassKey k{law, d.recon, d.riemann, (d.law != MARA_LAW_HYDRO && d.field_ct) ? 1 : 0,
-                     pencil, fused, pencil ? 1 : (express ? 2 : 0)};
+                     pencil, fused, pencil ? 1 : (express ? 2 : (fused == 1 || fused == 2 ? LANE_HYDRO : 0))};
     for (size_t c = 0; c < B->classes.size(); ++c)
         if (!(B->classes[c] < k) && !(k < B->classes[c])) return (int)c;
     B->classes.push_back(k);
@@ -374,6 +383,8 @@ int mara_batch_create(long long hbm_budget, int rk_order, int precision, int max
     if (!hip_ok(hipEventCreateWithFlags(&B->fork, hipEventDisableTiming))) return fail(MARA_ERR_HIP);
     if (!hip_ok(hipEventCreateWithFlags(&B->join, hipEventDisableTiming))) return fail(MARA_ERR_HIP);
     if (!hip_ok(hipEventCreateWithFlags(&B->join3, hipEventDisableTiming))) return fail(MARA_ERR_HIP);
+    if (!hip_ok(hipStreamCreateWithFlags(&B->stream4, hipStreamNonBlocking))) return fail(MARA_ERR_HIP);
+    if (!hip_ok(hipEventCreateWithFlags(&B->join4, hipEventDisableTiming))) return fail(MARA_ERR_HIP);
     if (!hip_ok(hipMalloc(&B->pool_mem, hbm_budget))) return fail(MARA_ERR_CAPACITY);
     B->pool.init(B->pool_mem, hbm_budget);
     if (!hip_ok(hipMalloc(&B->d_items, max_solves * sizeof(BItem)))) return fail(MARA_ERR_HIP);
@@ -394,6 +405,7 @@ int mara_batch_destroy(mara_batch* B)
     if (B->stream) (void)hipStreamSynchronize(B->stream);
     if (B->stream2) (void)hipStreamSynchronize(B->stream2);
     if (B->stream3) (void)hipStreamSynchronize(B->stream3);
+    if (B->stream4) (void)hipStreamSynchronize(B->stream4);
     (void)hipFree(B->pool_mem);
     (void)hipFree(B->d_items);
     (void)hipFree(B->d_ctl);
@@ -404,7 +416,7 @@ int mara_batch_destroy(mara_batch* B)
     (void)hipFree(B->d_src[0]);
     (void)hipFree(B->d_src[1]);
     if (B->src_module) (void)hipModuleUnload(B->src_module);
-    if (B->round_exec) (void)hipGraphExecDestroy(B->round_exec);
+    drop_graphs(B);
     if (B->h_ctl) (void)hipHostFree(B->h_ctl);
     if (B->stream) (void)hipStreamDestroy(B->stream);
     if (B->stream2) (void)hipStreamDestroy(B->stream2);
@@ -412,6 +424,8 @@ int mara_batch_destroy(mara_batch* B)
     if (B->fork) (void)hipEventDestroy(B->fork);
     if (B->join) (void)hipEventDestroy(B->join);
     if (B->join3) (void)hipEventDestroy(B->join3);
+    if (B->stream4) (void)hipStreamDestroy(B->stream4);
+    if (B->join4) (void)hipEventDestroy(B->join4);
     delete B;
     return MARA_OK;
 }
@@ -432,11 +446,7 @@ int mara_batch_set_source(mara_batch* B, const char* code_object, const char* ke
     B->src_zones = 0;
     B->classes.clear();  // class keys depend on whether a source is set
     B->dirty = true;
-    if (B->round_exec)
-    {
-        (void)hipGraphExecDestroy(B->round_exec);
-        B->round_exec = nullptr;
-    }
+    drop_graphs(B);
     if (!code_object) return MARA_OK;
     if (hipModuleLoad(&B->src_module, code_object) != hipSuccess)
     {
@@ -483,12 +493,8 @@ int mara_batch_set_source_aux(mara_batch* B, const double* t)
 int mara_batch_set_persistent(mara_batch* B, int workgroups_per_cu)
 {
     if (!B || workgroups_per_cu < 0 || workgroups_per_cu > 16) return MARA_ERR_INVALID_ARGUMENT;
-    if (B->persistent != workgroups_per_cu && B->round_exec)
-    {
-        // the captured round holds the other launches
-        (void)hipGraphExecDestroy(B->round_exec);
-        B->round_exec = nullptr;
-    }
+    // the captured rounds hold the other launches
+    if (B->persistent != workgroups_per_cu) drop_graphs(B);
     B->persistent = workgroups_per_cu;
     return MARA_OK;
 }
@@ -503,7 +509,8 @@ int mara_batch_set_express(mara_batch* B, int max_solves)
 int mara_batch_lane(const mara_batch* B, int slot, int* lane)
 {
     if (!B || !lane || slot < 0 || slot >= B->max_solves || !B->slots[slot].used) return MARA_ERR_INVALID_ARGUMENT;
-    *lane = B->items[slot].lane == LANE_CHIP ? 1 : B->items[slot].lane;
+    const int l = B->items[slot].lane;
+    *lane = l == LANE_CHIP ? 1 : l == LANE_HYDRO ? 0 : l;
     return MARA_OK;
 }
 
@@ -633,12 +640,8 @@ int mara_batch_admit(mara_batch* B, const mara_desc* d, const double* P, double 
         source_records(B, n, true);
         if (upload_source_records(B, n, 1)) return undo();
         B->src_zones = std::max(B->src_zones, (long long)it.G.n[0] * it.G.n[1] * it.G.n[2]);
-        if (B->round_exec)
-        {
-            // the captured round's source launch covers the old slot count and zone count
-            (void)hipGraphExecDestroy(B->round_exec);
-            B->round_exec = nullptr;
-        }
+        // the captured rounds' source launch covers the old slot count and zone count
+        drop_graphs(B);
     }
     // the host buffer may go away after return
     if (!hip_ok(hipStreamSynchronize(B->stream))) return undo();
@@ -697,8 +700,8 @@ int mara_batch_step(mara_batch* B, int n_steps, int* n_active)
     // tile-lane step; the other lanes take `ratio` / `ratio3` steps in it,
     // sized from the tile lane's estimated step time (its active zones at
     // ~5e9 zone-stages per second, plus ~20 us of launches) against theirs.
-    long long zones[4] = {0, 0, 0, 0};
-    bool busy[4] = {false, false, false, false};
+    long long zones[LANES_ALL] = {};
+    bool busy[LANES_ALL] = {};
     for (int k = 0; k < n; ++k)
     {
         if (!B->slots[k].used || finished(B->h_ctl[k])) continue;
@@ -706,7 +709,9 @@ int mara_batch_step(mara_batch* B, int n_steps, int* n_active)
         busy[l] = true;
         zones[l] += (long long)B->items[k].G.n[0] * B->items[k].G.n[1] * B->items[k].G.n[2];
     }
-    const bool any_tile = busy[0], any_pencil = busy[1], any_express = busy[2];
+    const bool any_hydro = busy[LANE_HYDRO], any_tile = busy[0] || any_hydro, any_pencil = busy[1],
+               any_express = busy[2];
+    zones[0] += zones[LANE_HYDRO];
     auto step_time = [&](int l) { return (double)zones[l] * B->rk_order / 5e9 + 20e-6; };
     const double round_time = any_tile ? step_time(0) : any_express ? step_time(2) : 20e-6;
     int ratio = 1, ratio3 = 1;
@@ -724,115 +729,89 @@ int mara_batch_step(mara_batch* B, int n_steps, int* n_active)
         chip_steps = n_steps * (int)std::min(32.0, std::max(1.0, fit));
     }
     const unsigned sg = (unsigned)((n + 3) / 4);  // kb_step_start: 4 items per work-group
-    // `count` steps of one lane: one kernel ends a step and starts the next
-    auto run_lane = [&](int lane, int count) {
-        kb_step_start<<<sg, 256, 0, B->cur>>>(B->d_items, n, lane);
+    // The lanes with work, each on its stream, and their steps in a round.  They
+    // share no data, so nothing orders them against each other inside a call.
+    struct Lane
+    {
+        int lane, count;
+        hipStream_t stream;
+    };
+    std::vector<Lane> lanes;
+    if (busy[0] || (!any_tile && !any_pencil && !any_express && !chip_steps)) lanes.push_back({0, 1, B->stream});
+    if (any_hydro) lanes.push_back({LANE_HYDRO, 1, B->stream4});
+    if (any_pencil) lanes.push_back({1, ratio, B->stream2});
+    if (any_express) lanes.push_back({2, ratio3, B->stream3});
+    // `count` steps of a lane, the first of a call or not, the last or not: one
+    // kernel ends a step and starts the next
+    const auto run_lane = [&](const Lane& l, int count, bool first, bool last) {
+        B->cur = l.stream;
+        if (first) kb_step_start<<<sg, 256, 0, B->cur>>>(B->d_items, n, l.lane);
         for (int s = 0; s < count; ++s)
         {
             for (int rk = 0; rk < B->rk_order; ++rk)
             {
-                if (B->precision == MARA_PREC_MIXED) run_stage_f32(B, rk, lane);
-                else run_stage<double>(B, rk, lane);
+                if (B->precision == MARA_PREC_MIXED) run_stage_f32(B, rk, l.lane);
+                else run_stage<double>(B, rk, l.lane);
             }
-            if (s + 1 < count) kb_step_next<<<sg, 256, 0, B->cur>>>(B->d_items, n, lane);
-            else kb_step_end<<<ig, 64, 0, B->cur>>>(B->d_items, n, lane);
+            if (s + 1 < count || !last) kb_step_next<<<sg, 256, 0, B->cur>>>(B->d_items, n, l.lane);
+            else kb_step_end<<<ig, 64, 0, B->cur>>>(B->d_items, n, l.lane);
         }
     };
-    auto run_round = [&]() {
-        if (any_tile || (!any_pencil && !any_express && !chip_steps))
+    // A lane's round as a graph of its own (one chain of kernels: a graph with a
+    // branch per lane leaves 30 to 50 us between rounds), captured in the second
+    // call with the same solves: a capture costs about 0.1 ms per kernel, which
+    // a set that changes with every call never earns back.
+    const bool replay = B->graphs && n > 0 && n_steps > 1 && B->last_version == B->table_version;
+    B->last_version = B->table_version;
+    if (replay)
+        for (const Lane& l : lanes)
         {
-            B->cur = B->stream;
-            run_lane(0, 1);
-        }
-        if (any_pencil)
-        {
-            B->cur = B->stream2;
-            run_lane(1, ratio);
-        }
-        if (any_express)
-        {
-            B->cur = B->stream3;
-            run_lane(2, ratio3);
-        }
-    };
-    const int lanes = (any_tile ? 1 : 0) | (any_pencil ? 2 : 0) | (any_express ? 4 : 0);
-    // beside the rounds, from where the first stream stands
-    const auto launch_chips = [&]() {
-        HIP_TRY(hipEventRecord(B->fork, B->stream));
-        HIP_TRY(hipStreamWaitEvent(B->stream2, B->fork, 0));
-        HIP_TRY(hipStreamWaitEvent(B->stream3, B->fork, 0));
-        for (const ChipSegment& s : B->chip_segments)
-        {
-            const hipStream_t to = B->classes[s.cls].law == MARA_LAW_HYDRO ? B->stream2 : B->stream3;
-            B->precision == MARA_PREC_MIXED ? run_chip_f32(B, s, chip_steps, to) : run_chip<double>(B, s, chip_steps, to);
-        }
-        HIP_TRY(hipEventRecord(B->join, B->stream2));
-        HIP_TRY(hipEventRecord(B->join3, B->stream3));
-        return (int)MARA_OK;
-    };
-    const auto join_chips = [&]() {
-        HIP_TRY(hipStreamWaitEvent(B->stream, B->join, 0));
-        HIP_TRY(hipStreamWaitEvent(B->stream, B->join3, 0));
-        return (int)MARA_OK;
-    };
-    if (chip_steps && !lanes)
-    {
-        if (launch_chips() || join_chips()) return MARA_ERR_HIP;
-    }
-    else if (B->graphs && n > 0 && n_steps > 1)
-    {
-        if (!B->round_exec || B->round_version != B->table_version || B->round_n != n || B->round_ratio != ratio
-            || B->round_ratio3 != ratio3 || B->round_lanes != lanes)
-        {
-            if (B->round_exec) HIP_TRY(hipGraphExecDestroy(B->round_exec));
-            B->round_exec = nullptr;
-            // the round forks the other streams off the first and joins them
-            // back, so one replay ends when every lane has
+            LaneGraph& lg = B->lane_graph[l.lane];
+            if (lg.exec && lg.version == B->table_version && lg.n == n && lg.count == l.count) continue;
+            if (lg.exec) HIP_TRY(hipGraphExecDestroy(lg.exec));
+            lg.exec = nullptr;
             hipGraph_t g = nullptr;
-            HIP_TRY(hipStreamBeginCapture(B->stream, hipStreamCaptureModeThreadLocal));
-            (void)hipEventRecord(B->fork, B->stream);
-            (void)hipStreamWaitEvent(B->stream2, B->fork, 0);
-            (void)hipStreamWaitEvent(B->stream3, B->fork, 0);
-            run_round();
-            (void)hipEventRecord(B->join, B->stream2);
-            (void)hipEventRecord(B->join3, B->stream3);
-            (void)hipStreamWaitEvent(B->stream, B->join, 0);
-            (void)hipStreamWaitEvent(B->stream, B->join3, 0);
+            HIP_TRY(hipStreamBeginCapture(l.stream, hipStreamCaptureModeThreadLocal));
+            run_lane(l, l.count, true, true);
             const hipError_t launched = hipGetLastError();
-            const hipError_t ended = hipStreamEndCapture(B->stream, &g);
+            const hipError_t ended = hipStreamEndCapture(l.stream, &g);
             if (!hip_ok(launched) || !hip_ok(ended))
             {
                 if (g) (void)hipGraphDestroy(g);
                 return MARA_ERR_HIP;
             }
-            const hipError_t made = hipGraphInstantiate(&B->round_exec, g, nullptr, nullptr, 0);
+            const hipError_t made = hipGraphInstantiate(&lg.exec, g, nullptr, nullptr, 0);
             (void)hipGraphDestroy(g);
             if (!hip_ok(made))
             {
-                B->round_exec = nullptr;
+                lg.exec = nullptr;
                 return MARA_ERR_HIP;
             }
-            B->round_version = B->table_version;
-            B->round_n = n;
-            B->round_ratio = ratio;
-            B->round_ratio3 = ratio3;
-            B->round_lanes = lanes;
+            lg.version = B->table_version;
+            lg.n = n;
+            lg.count = l.count;
         }
-        if (chip_steps && launch_chips()) return MARA_ERR_HIP;
-        for (int s = 0; s < n_steps; ++s) HIP_TRY(hipGraphLaunch(B->round_exec, B->stream));
-        if (chip_steps && join_chips()) return MARA_ERR_HIP;
-    }
-    else
+    // every stream from where the first one stands, and back
+    const hipStream_t side[3] = {B->stream2, B->stream3, B->stream4};
+    const hipEvent_t back[3] = {B->join, B->join3, B->join4};
+    HIP_TRY(hipEventRecord(B->fork, B->stream));
+    for (hipStream_t st : side) HIP_TRY(hipStreamWaitEvent(st, B->fork, 0));
+    if (chip_steps)
+        for (const ChipSegment& s : B->chip_segments)
+        {
+            const hipStream_t to = B->classes[s.cls].law == MARA_LAW_HYDRO ? B->stream2 : B->stream3;
+            B->precision == MARA_PREC_MIXED ? run_chip_f32(B, s, chip_steps, to) : run_chip<double>(B, s, chip_steps, to);
+        }
+    for (int s = 0; s < n_steps && n > 0; ++s)
+        for (const Lane& l : lanes)
+        {
+            if (replay) HIP_TRY(hipGraphLaunch(B->lane_graph[l.lane].exec, l.stream));
+            else run_lane(l, l.count, s == 0, s + 1 == n_steps);
+        }
+    for (int k = 0; k < 3; ++k)
     {
-        HIP_TRY(hipEventRecord(B->fork, B->stream));
-        HIP_TRY(hipStreamWaitEvent(B->stream2, B->fork, 0));
-        HIP_TRY(hipStreamWaitEvent(B->stream3, B->fork, 0));
-        if (chip_steps && launch_chips()) return MARA_ERR_HIP;
-        for (int s = 0; s < n_steps && n > 0; ++s) run_round();
-        HIP_TRY(hipEventRecord(B->join, B->stream2));
-        HIP_TRY(hipEventRecord(B->join3, B->stream3));
-        HIP_TRY(hipStreamWaitEvent(B->stream, B->join, 0));
-        HIP_TRY(hipStreamWaitEvent(B->stream, B->join3, 0));
+        HIP_TRY(hipEventRecord(back[k], side[k]));
+        HIP_TRY(hipStreamWaitEvent(B->stream, back[k], 0));
     }
     HIP_TRY(hipGetLastError());
     if (n) HIP_TRY(hipMemcpyAsync(B->h_ctl, B->d_ctl, n * sizeof(Ctl), hipMemcpyDeviceToHost, B->stream));

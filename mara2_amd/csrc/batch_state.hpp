@@ -87,7 +87,7 @@ struct ClassKey
     int law, recon, riemann, ct;
     int pencil;  // 1-D items of an RK2 batch: fused pencil tiles
     int fused;   // RK2 batch fused stage tiles: hydro + PLM on 2-D (1) or 3-D (2) meshes, MHD on 2-D (3)
-    int lane;    // 0 tile lane, 1 pencil lane, 2 express lane (long chains)
+    int lane;    // 0 tile lane, 1 pencil lane, 2 express lane (long chains), LANE_HYDRO
     bool operator<(const ClassKey& o) const
     {
         return std::tie(law, recon, riemann, ct, pencil, fused, lane)
@@ -109,6 +109,21 @@ struct ChipSegment
 constexpr int CHIP_RESIDENT = 224;
 // lane of the solves that run on chip (mara_batch_lane reports the pencil lane, 1)
 constexpr int LANE_CHIP = 3;
+// lane of the 2-D and 3-D hydro tiles, beside the tile lane's other solves on
+// a stream of its own: the two share no data, and one lane's kernels fill the
+// CUs that the last round of the other's tiles leaves empty (reported as the
+// tile lane, 0)
+constexpr int LANE_HYDRO = 4;
+constexpr int LANES_ALL = 5;
+
+// HIP graph of one lane's steps in a round, replayed n_steps times by
+// mara_batch_step; recaptured when the table, the slot count or the steps change
+struct LaneGraph
+{
+    hipGraphExec_t exec = nullptr;
+    long long version = -1;
+    int n = -1, count = -1;
+};
 
 } // namespace batch
 } // namespace mara
@@ -141,8 +156,9 @@ struct mara_batch
     hipStream_t stream = nullptr;   // tile kernels, transfers, control
     hipStream_t stream2 = nullptr;  // pencil kernels of 1-D solves
     hipStream_t stream3 = nullptr;  // express lane: the longest chains of 2-D/3-D solves
+    hipStream_t stream4 = nullptr;  // hydro tiles
     hipStream_t cur = nullptr;      // stream the stage launches go to
-    hipEvent_t fork = nullptr, join = nullptr, join3 = nullptr;
+    hipEvent_t fork = nullptr, join = nullptr, join3 = nullptr, join4 = nullptr;
     mara::batch::Pool pool;
     char* pool_mem = nullptr;
     mara::BItem* d_items = nullptr;
@@ -166,13 +182,9 @@ struct mara_batch
     mara::BChip* d_chips = nullptr;
     int chip_capacity = 0;
     long long table_version = 0;                   // bumped by every table build
-    // HIP graph of one round (a tile-lane step and `ratio` pencil-lane steps),
-    // replayed n_steps times by mara_batch_step; recaptured when the table,
-    // the slot count, the ratio or the set of busy lanes changes
     bool graphs = true;
-    hipGraphExec_t round_exec = nullptr;
-    long long round_version = -1;
-    int round_n = -1, round_ratio = -1, round_ratio3 = -1, round_lanes = -1;
+    mara::batch::LaneGraph lane_graph[mara::batch::LANES_ALL];
+    long long last_version = -1;  // table_version of the last call of mara_batch_step
 };
 
 namespace mara {
