@@ -32,20 +32,6 @@ constexpr int FUSED_KZ = 16;  // default z planes per work-group (a launch shape
 constexpr int KZ_SHAPES[4] = {4, 8, 16, 32};  // the tuner's fixed candidates
 constexpr int KZ_MAX = 1024;                   // set_shape accepts 1 .. KZ_MAX
 
-// Work-group -> tile order that keeps neighbouring tiles on one XCD.  The
-// dispatcher hands work-group L of a 1-D grid to XCD L % 8, and each XCD has
-// its own L2.  Tiles [start(x), start(x + 1)) in x-fastest order go to XCD x,
-// in launch order, so tiles that share halo rows and columns run side by side
-// behind the same L2.  The map is a bijection on [0, ntiles).
-constexpr int NUM_XCD = 8;
-
-__device__ __forceinline__ int xcd_tile(int L, int ntiles)
-{
-    const int x = L % NUM_XCD, l = L / NUM_XCD;
-    const int q = ntiles / NUM_XCD, r = ntiles % NUM_XCD;
-    return x * q + (x < r ? x : r) + l;
-}
-
 // Whole-wavefront lane shifts by one through DPP (wave_shr:1 / wave_shl:1 on
 // every dword): lane l takes v of lane l - 1 (shift_up) or l + 1
 // (shift_down), and the lane with no source, 0 or 63, keeps `edge` (bound_ctrl

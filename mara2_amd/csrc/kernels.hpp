@@ -187,6 +187,35 @@ __device__ __forceinline__ T wave_max(T v)
 }
 
 
+// Work-group -> tile order that keeps neighbouring tiles on one XCD.  The
+// dispatcher hands work-group L of a 1-D grid to XCD L % 8, and each XCD has
+// its own L2.  Tiles [start(x), start(x + 1)) in x-fastest order go to XCD x,
+// in launch order, so tiles that share halo rows and columns run side by side
+// behind the same L2.  The map is a bijection on [0, ntiles).
+constexpr int NUM_XCD = 8;
+
+__device__ __forceinline__ int xcd_tile(int L, int ntiles)
+{
+    const int x = L % NUM_XCD, l = L / NUM_XCD;
+    const int q = ntiles / NUM_XCD, r = ntiles % NUM_XCD;
+    return x * q + (x < r ? x : r) + l;
+}
+
+// The work-group of a box of (gx, gy, gz) work-groups that a 1-D grid's
+// work-group takes in that order: an XCD gets whole z slabs, so the planes its
+// z stencils and flux-CT gathers share are in its own L2.
+struct BoxGroup
+{
+    int x, y, z;
+};
+
+__device__ __forceinline__ BoxGroup box_group(int gx, int gy)
+{
+    const unsigned L = (unsigned)xcd_tile((int)blockIdx.x, (int)gridDim.x);
+    const unsigned row = L / (unsigned)gx;
+    return {(int)(L - row * (unsigned)gx), (int)(row % (unsigned)gy), (int)(row / (unsigned)gy)};
+}
+
 // ---------------------------------------------------------------------------
 // Face flux sweep: MeshOperator::godunov + the IntercellFluxScheme
 // (src/MeshOperator.cpp:443-525, src/IntercellFluxSchemes.cpp:45-117).
@@ -349,7 +378,7 @@ k_flux(const double* __restrict__ P, R* __restrict__ F, const Geom G, int axis,
     int ti, tj, tk;
     if (linear)
     {
-        const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
+        const unsigned t = (unsigned)xcd_tile((int)blockIdx.x, (int)gridDim.x) * blockDim.x + threadIdx.x;
         const unsigned row = t / (unsigned)m0;
         ti = (int)(t - row * (unsigned)m0);
         tj = (int)(row % (unsigned)m1);
@@ -358,9 +387,10 @@ k_flux(const double* __restrict__ P, R* __restrict__ F, const Geom G, int axis,
     }
     else
     {
-        ti = blockIdx.x * blockDim.x + threadIdx.x;
-        tj = blockIdx.y * blockDim.y + threadIdx.y;
-        tk = (int)blockIdx.z;
+        const BoxGroup b = box_group((m0 + 63) / 64, (m1 + (int)blockDim.y - 1) / (int)blockDim.y);
+        ti = b.x * 64 + threadIdx.x;
+        tj = b.y * blockDim.y + threadIdx.y;
+        tk = b.z;
         if (ti >= m0 || tj >= m1) return;
     }
     flux_face<Law, Recon, Riem, R, AX>(P, F, G, AX < 0 ? axis : AX, lo0 + ti, lo1 + tj, lo2 + tk, ctl);
@@ -928,12 +958,13 @@ k_update(const double* __restrict__ P0, double* __restrict__ U, double* __restri
 {
     __shared__ double wmin[4];
     if (!ctl->active) return;
-    const int ti = blockIdx.x * blockDim.x + threadIdx.x;
-    const int tj = blockIdx.y * blockDim.y + threadIdx.y;
+    const BoxGroup bg = box_group((G.n[0] + 63) / 64, (G.n[1] + (int)blockDim.y - 1) / (int)blockDim.y);
+    const int ti = bg.x * 64 + threadIdx.x;
+    const int tj = bg.y * blockDim.y + threadIdx.y;
     double dtc = 1.79769313486231570815e+308;
     if (ti < G.n[0] && tj < G.n[1])
         dtc = update_zone<Law, R, CT>(P0, U, Pout, Fx, Fy, Fz, G, b, first_stage, write_u, courant_out, ctl,
-                                      G.g[0] + ti, G.g[1] + tj, G.g[2] + (int)blockIdx.z, Ssrc);
+                                      G.g[0] + ti, G.g[1] + tj, G.g[2] + bg.z, Ssrc);
     if (courant_out) courant_to_bins(dtc, wmin, (int)blockDim.y, threadIdx.y * blockDim.x + threadIdx.x, ctl);
 }
 

@@ -51,13 +51,13 @@ struct StageArgs
     void* after_flux_ctx;
 };
 
-// 2-D work-groups of 64 x rows over an (m0, m1, m2) box: one wavefront per x
-// row, z from the grid, so kernels decode indices without integer division.
+// 2-D work-groups of 64 x rows over an (m0, m1, m2) box, one wavefront per x
+// row, on a 1-D grid that box_group orders by XCD.
 // rows (1, 2 or 4) is a launch shape; the result does not depend on it.
 constexpr int ROWS_DEFAULT = 4;
 constexpr int ROWS_SHAPES[3] = {1, 2, 4};
 inline dim3 stage_block3(int rows) { return dim3(64, rows, 1); }
-inline dim3 stage_grid3(int m0, int m1, int m2, int rows) { return dim3((m0 + 63) / 64, (m1 + rows - 1) / rows, m2); }
+inline dim3 stage_grid3(int m0, int m1, int m2, int rows) { return dim3((m0 + 63) / 64 * ((m1 + rows - 1) / rows) * m2); }
 
 template <int Law, int Recon, int Riem, typename R, int AX>
 void flux_sweep(const StageArgs& s, int axis, const int* lo, const int* hi)
