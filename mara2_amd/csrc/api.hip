@@ -335,16 +335,16 @@ void launch_stage(mara_block* b, int rk, int courant_out)
         hipEventRecord(b->ev[2 * b->ev_used + 1], b->stream);
         b->ev_used += 1;
     }
-    // the flux-array update writes the ghost zones of Pout itself
-    // (write_guard_images); the fused kernels leave them to a ghost-fill pass,
-    // and a group member's guards come from the group's exchange after the
-    // stage (the images the update wrote are then overwritten).  The PLM
+    // the flux-array update and the 2-D tiles write the ghost zones of Pout
+    // themselves (write_guard_images); the 3-D tiles leave them to a ghost-fill
+    // pass, and a group member's guards come from the group's exchange after
+    // the stage (the images the update wrote are then overwritten).  The PLM
     // tiles of a periodic block read no guards: their output's are filled
     // when something reads them (fill_guards).
     if (b->fused && !b->in_group)
     {
-        if (!wrap) launch_bc(b, Pout);
-        else if (last) b->guards_stale = true;
+        if (wrap) b->guards_stale = b->guards_stale || last;
+        else if (b->G.N[2] > 1) launch_bc(b, Pout);
     }
 }
 

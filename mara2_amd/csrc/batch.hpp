@@ -172,7 +172,7 @@ kb_fused_plm(const BItem* __restrict__ items, const BTile* __restrict__ tiles, d
     const double* Pin = first ? it.Pa : it.Pb;
     double* Pout = last ? it.Pa : it.Pb;
     fused_plm_tile<Riem, R, Z>(Pin, it.Pa, it.U, Pout, G, b, first, !last, courant_out, it.ctl, T.x0, T.y0, T.z0,
-                               kz, false);
+                               kz, false, false);
 }
 
 // The mixed form's 2-D and 3-D hydro + PLM items: the single block's tiles
@@ -190,7 +190,7 @@ kb_fast_plm(const BItem* __restrict__ items, const BTile* __restrict__ tiles, do
     const double* Pin = first ? it.Pa : it.Pb;
     double* Pout = last ? it.Pa : it.Pb;
     fast64::fast_plm_tile<float, Riem, Z>(Pin, it.Pa, Pout, G, b, first, courant_out, it.ctl, T.x0, T.y0, T.z0, kz,
-                                          false);
+                                          false, false);
 }
 
 // ---------------------------------------------------------------------------
@@ -238,7 +238,7 @@ kbq_fused_plm(const BItem* __restrict__ items, const BTile* __restrict__ tiles, 
         const double* Pin = first ? it.Pa : it.Pb;
         double* Pout = last ? it.Pa : it.Pb;
         fused_plm_tile<Riem, R, Z>(Pin, it.Pa, it.U, Pout, it.G, b, first, !last, courant_out, it.ctl, T.x0, T.y0,
-                                   T.z0, kz, false);
+                                   T.z0, kz, false, false);
     }
 }
 
@@ -257,7 +257,7 @@ kbq_fast_plm(const BItem* __restrict__ items, const BTile* __restrict__ tiles, i
         const double* Pin = first ? it.Pa : it.Pb;
         double* Pout = last ? it.Pa : it.Pb;
         fast64::fast_plm_tile<float, Riem, Z>(Pin, it.Pa, Pout, it.G, b, first, courant_out, it.ctl, T.x0, T.y0,
-                                              T.z0, kz, false);
+                                              T.z0, kz, false, false);
     }
 }
 

@@ -224,7 +224,7 @@ template <typename R, int Riem, bool Z>
 __device__ __forceinline__ void fast_plm_tile(const double* __restrict__ Pin, const double* __restrict__ P0,
                                               double* __restrict__ Pout, const Geom& G, double b, int first_stage,
                                               int courant_out, Ctl* ctl, int tx, int ty, int tz, int kz,
-                                              bool wrap)
+                                              bool wrap, bool images)
 {
     constexpr bool F64 = sizeof(R) == 8;
     constexpr int NG = 2, TX = FastTile<R>::TX, TY = FastTile<R>::TY;
@@ -486,6 +486,8 @@ __device__ __forceinline__ void fast_plm_tile(const double* __restrict__ Pin, co
             prim_of(gm1, Un, Pn);
 #pragma unroll
             for (int q = 0; q < 5; ++q) __builtin_nontemporal_store(Pn[q], &Pout[q * G.fs + c]);
+            if constexpr (!Z)
+                if (images) write_guard_images<5>(Pout, G, i, j, k, Pn);
             if (courant_out)
             {
                 const double d = courant(K, Pn, G.Lmin);
@@ -518,7 +520,8 @@ k_fast_plm(const double* __restrict__ Pin, const double* __restrict__ P0, double
     const int ntz = Z ? (G.n[2] + kz - 1) / kz : 1;
     const int tile = xcd_tile(blockIdx.x, ntx * nty * ntz);
     const int tx = tile % ntx, ty = (tile / ntx) % nty, tz = tile / (ntx * nty);
-    fast_plm_tile<R, Riem, Z>(Pin, P0, Pout, G, b, first_stage, courant_out, ctl, tx, ty, tz, kz, wrap != 0);
+    fast_plm_tile<R, Riem, Z>(Pin, P0, Pout, G, b, first_stage, courant_out, ctl, tx, ty, tz, kz, wrap != 0,
+                              wrap == 0);
 }
 
 // the blocks this kernel serves: hydro, PLM, 2-D or 3-D, two or three stages
