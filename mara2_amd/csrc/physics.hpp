@@ -425,8 +425,55 @@ __device__ __forceinline__ void mhd_state(R gamma, const R* P, const R* dAA, Sta
     S.A[7] = vn + sF;
 }
 
+// The smallest and largest root of k4 x^4 + ... + k0 with four real roots, by
+// Newton's method on both at once from mid -+ half.  Taken only where it is
+// sure: both starts lie outside every real root (no Taylor coefficient there
+// points inwards), so the iteration falls towards the outermost one without
+// overshooting; both steps end below 1e-8 half, whose square is the error
+// left; and neither root is near a second one (a slope of 1e-5 k4 half^3 at
+// least, where the roots' own error is that of rounding).  False elsewhere:
+// double or complex roots, and starts that are not numbers.
+__device__ __forceinline__ bool outermost_roots(double k4, double k3, double k2, double k1, double k0, double mid,
+                                                double half, double& lo, double& hi)
+{
+#pragma clang fp contract(fast)
+    const double d3 = 4.0 * k4, d2 = 3.0 * k3, d1 = 2.0 * k2;
+    lo = mid - half;
+    hi = mid + half;
+    // second derivative (half of it) positive, third (a sixth) outwards; value
+    // and slope in the first iteration
+    const bool convex = (6.0 * k4 * lo + d2) * lo + k2 > 0.0 && (6.0 * k4 * hi + d2) * hi + k2 > 0.0
+        && d3 * lo + k3 < 0.0 && d3 * hi + k3 > 0.0;
+    if (!(k4 > 0.0 && convex)) return false;
+    const double settled = 1e-8 * half;
+    const double slope = 1e-5 * k4 * (half * half) * half;
+    for (int n = 0; n < 12; ++n)
+    {
+        const double fl = (((k4 * lo + k3) * lo + k2) * lo + k1) * lo + k0;
+        const double fh = (((k4 * hi + k3) * hi + k2) * hi + k1) * hi + k0;
+        const double gl = ((d3 * lo + d2) * lo + d1) * lo + k1;
+        const double gh = ((d3 * hi + d2) * hi + d1) * hi + k1;
+        // the hardware reciprocal's 2^-23 is 2^-23 of a step, and the last one
+        // is below 1e-8 half
+        const double sl = fl * __builtin_amdgcn_rcp(gl), sh = fh * __builtin_amdgcn_rcp(gh);
+        if (n == 0 && !(sl < settled && sh > -settled && gl < 0.0 && gh > 0.0)) return false;
+        lo -= sl;
+        hi -= sh;
+        if (__builtin_fabs(sl) < settled && __builtin_fabs(sh) < settled) return gl < -slope && gh > slope;
+    }
+    return false;
+}
+
 // RelativisticMHD eigenvalues (src/ConservationLaws.cpp:739-835), binary64.
-// Returns ERR_NONE or ERR_EIGEN.
+// Returns ERR_NONE or ERR_EIGEN.  The Riemann solver and the CFL time step
+// read the outermost eigenvalues only, so the quartic's inner roots are not
+// sought where its outer ones settle (A[2] and A[5] then hold v_n, which lies
+// between); the start is the fast speed of a field without direction,
+// a^2 = cs^2 + ca^2 - cs^2 ca^2, which bounds the fast speed of every
+// direction.  Elsewhere all real roots come from Ferrari's method, whose cubic
+// takes an arc cosine and a cosine or two cube roots.  Two to four iterations
+// are usual, and the speeds are at least as close (rounding, where Ferrari's
+// coefficients can cancel).  Flux sweep at 128^3: 205 -> 192 us.
 __device__ inline int rmhd_eigen(double gamma, const double* P, const double* dAA, double* A)
 {
 #pragma clang fp contract(fast)
@@ -467,9 +514,27 @@ __device__ inline int rmhd_eigen(double gamma, const double* P, const double* dA
     const double A2 = 6 * K * v2 + L * (1. - v2) + b0 * b0 - bn * bn;
     const double A1 = -4 * K * v3 - L * vn * 2 - 2 * b0 * bn;
     const double A0 = K * v4 + L * v2 + bn * bn;
+    const double C = Rel::sqrt(h0 + bb);
+    const double ca2 = Rel::div_pos(bb, P[0] * h0 + bb);
+    const double a2 = cs2 + ca2 - cs2 * ca2;
+    const double den = Rel::div_pos(1.0, 1.0 - vv * a2);
+    const double mid = vn * (1.0 - a2) * den;
+    const double half = Rel::sqrt(a2 * (1.0 - vv) * ((1.0 - vv * a2) - v2 * (1.0 - a2))) * den;
+    double lo, hi;
+    if (outermost_roots(A4, A3, A2, A1, A0, mid, half, lo, hi))
+    {
+        A[0] = lo;
+        A[1] = Rel::div(bn - C * vn * W0, b0 - C * W0);
+        A[2] = vn;
+        A[3] = vn;
+        A[4] = vn;
+        A[5] = vn;
+        A[6] = Rel::div(bn + C * vn * W0, b0 + C * W0);
+        A[7] = hi;
+        return ERR_NONE;
+    }
     double roots[4];
     const int nr = quartic_real_roots(A4, A3, A2, A1, A0, roots);
-    const double C = Rel::sqrt(h0 + bb);
     if (nr == 4)
     {
         A[0] = roots[0];
