@@ -396,6 +396,86 @@ k_flux(const double* __restrict__ P, R* __restrict__ F, const Geom G, int axis,
     flux_face<Law, Recon, Riem, R, AX>(P, F, G, AX < 0 ? axis : AX, lo0 + ti, lo1 + tj, lo2 + tk, ctl);
 }
 
+// The relativistic WENO5 sweep in binary64.  It is bound by its arithmetic, a
+// third of which weighs the candidate stencils, and a zone's two edges take
+// the same weights: here a thread reconstructs both edges of one zone, hands
+// the right one to its neighbour through LDS, and solves the zone's left face.
+// Along x a work-group is a run of zones in x-fastest order, whose first lane
+// only reconstructs; along y and z it is WENO_ACROSS positions across the axis
+// (a 128 B line each) by WENO_ALONG zones along it, whose first row only
+// reconstructs.  Sweeps at 128^3: 192 -> 158, 176 and 172 us.  Along y and z 64
+// positions by 4 zones took 196 and 192 (a third more reconstructions than
+// zones), 8 by 32 188 and 184 (129 faces fill five slabs of 31 less well than
+// nine of 15), and work-groups of 6 or 8 wavefronts 205 to 270 (at 144
+// registers three work-groups of 4 fit a compute unit).
+constexpr int WENO_ACROSS = 16, WENO_ALONG = 16, WENO_THREADS = WENO_ACROSS * WENO_ALONG;
+
+template <int AX>
+static __global__ void __launch_bounds__(WENO_THREADS)
+k_flux_weno(const double* __restrict__ P, double* __restrict__ F, const Geom G, int lo0, int lo1, int lo2, int m0,
+            int m1, int m2, Ctl* ctl)
+{
+    constexpr int NQ = LawNQ<2>::value;
+    __shared__ double edge[NQ][WENO_THREADS];
+    if (!ctl->active) return;
+    const unsigned tile = (unsigned)xcd_tile((int)blockIdx.x, (int)gridDim.x);
+    int i, j, k;      // the zone, and the face on its left
+    bool zone, face;  // whether the box has them
+    if constexpr (AX == 0)
+    {
+        const unsigned span = (unsigned)m0 + 1;
+        const unsigned t = tile * (WENO_THREADS - 1) + threadIdx.x;
+        const unsigned row = t / span, at = t - row * span;
+        i = lo0 - 1 + (int)at;
+        j = lo1 + (int)(row % (unsigned)m1);
+        k = lo2 + (int)(row / (unsigned)m1);
+        zone = k < lo2 + m2;
+        face = zone && at > 0 && threadIdx.x > 0;
+    }
+    else
+    {
+        const int m = AX == 1 ? m1 : m2, across = AX == 1 ? m2 : m1;
+        const unsigned blocks = (unsigned)(m + WENO_ALONG - 2) / (WENO_ALONG - 1);
+        const int row = (int)threadIdx.x / WENO_ACROSS;
+        const int at = (int)(tile % blocks) * (WENO_ALONG - 1) + row;
+        const unsigned c = tile / blocks * WENO_ACROSS + threadIdx.x % WENO_ACROSS;
+        const int o = (int)(c / (unsigned)m0);
+        i = lo0 + (int)(c % (unsigned)m0);
+        j = AX == 1 ? lo1 - 1 + at : lo1 + o;
+        k = AX == 2 ? lo2 - 1 + at : lo2 + o;
+        zone = o < across && at <= m;
+        face = zone && row > 0;
+    }
+    double PL[NQ], PR[NQ];
+    if (zone)
+    {
+        const long long stride = AX == 0 ? 1 : AX == 1 ? (long long)G.N[0] : (long long)G.N[0] * G.N[1];
+        const long long c0 = cell_index(G, i, j, k);
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+        {
+            // field by field, as face_flux_at does
+            const double* Pq = P + q * G.fs + c0;
+            double v[5];
+#pragma unroll
+            for (int n = 0; n < 5; ++n) v[n] = Pq[(n - 2) * stride];
+            const WenoWeights W = weno_weights(v[0], v[1], v[2], v[3], v[4]);
+            edge[q][threadIdx.x] = weno_edge<true>(W, v[0], v[1], v[2], v[3], v[4]);
+            PR[q] = weno_edge<false>(W, v[0], v[1], v[2], v[3], v[4]);
+            asm volatile("" : : "v"(PR[q]) : "memory");
+        }
+    }
+    __syncthreads();
+    if (!face) return;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) PL[q] = edge[q][threadIdx.x - (AX == 0 ? 1 : WENO_ACROSS)];
+    double Fq[NQ];
+    face_flux_lr<2, 0, double>(PL, PR, G, AX, Fq, ctl);
+    const long long f = face_index(G, i, j, k);
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) F[q * G.ffs + f] = Fq[q];
+}
+
 // ---------------------------------------------------------------------------
 // Flux-CT (CellCenteredFieldCT::correctGodunovFluxes, Toth 2000 eq. 25,
 // src/CellCenteredFieldCT.cpp:14-134).  For face axis a and transverse

@@ -76,6 +76,26 @@ void flux_sweep(const StageArgs& s, int axis, const int* lo, const int* hi)
             s.Pin, (R*)s.F[axis], G, axis, lo[0], lo[1], lo[2], m0, m1, m2, 0, s.ctl);
 }
 
+// One relativistic WENO5 sweep over the faces [lo, hi) with shared weights.
+// False, and nothing launched, where its work-groups would cover more than 6/5
+// of the faces: a face costs 158/192 of k_flux's there (128^3), so shorter
+// axes (fewer than 15 faces, 16 to 26, 31 to 39, ...) stay with k_flux.
+template <int AX>
+bool weno_sweep(const StageArgs& s, const int* lo, const int* hi)
+{
+    const long long m[3] = {hi[0] - lo[0], hi[1] - lo[1], hi[2] - lo[2]};
+    const long long slabs = (m[AX] + WENO_ALONG - 2) / (WENO_ALONG - 1);
+    const long long rows = AX == 0 ? m[0] + 1 : slabs * WENO_ALONG;
+    if (5 * rows > 6 * m[AX]) return false;
+    const long long zones = (m[0] + 1) * m[1] * m[2], across = m[0] * m[AX == 1 ? 2 : 1];
+    const long long groups = AX == 0 ? (zones - 2 + (WENO_THREADS - 1)) / (WENO_THREADS - 1)
+                                     : (across + WENO_ACROSS - 1) / WENO_ACROSS * slabs;
+    if (zones >= (1ll << 31)) return false;  // 32-bit positions
+    k_flux_weno<AX><<<(unsigned)groups, WENO_THREADS, 0, s.stream>>>(
+        s.Pin, (double*)s.F[AX], *s.G, lo[0], lo[1], lo[2], (int)m[0], (int)m[1], (int)m[2], s.ctl);
+    return true;
+}
+
 template <int Law, int Recon, int Riem, typename R>
 void stage_flux_t(const StageArgs& s, int axis)
 {
@@ -91,6 +111,11 @@ void stage_flux_t(const StageArgs& s, int axis)
             lo[a] = G.g[a] - ring;
             hi[a] = G.N[a] - G.g[a] + ring;
         }
+    }
+    if constexpr (Law == 2 && Recon == 2 && sizeof(R) == 8)
+    {
+        if (axis == 0 ? weno_sweep<0>(s, lo, hi) : axis == 1 ? weno_sweep<1>(s, lo, hi) : weno_sweep<2>(s, lo, hi))
+            return;
     }
     if constexpr (ReferenceForm<Law, R, LawMath<Law, R>>::value)
     {
