@@ -858,7 +858,7 @@ int mara_block_upload_prim(mara_block* b, const double* P)
     }
     else
         HIP_TRY(hipMemcpyAsync(b->U, P, bytes, hipMemcpyHostToDevice, b->stream));
-    k_aos_to_soa<<<grid_for(b->S.ncell), kThreads, 0, b->stream>>>(b->U, b->Pa, b->G);
+    launch_transpose<true>(b->U, b->Pa, b->G, b->stream);
     b->guards_stale = false;
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(b->stream));
@@ -870,7 +870,7 @@ int mara_block_download_prim(mara_block* b, double* P)
     if (!b || !P) return MARA_ERR_INVALID_ARGUMENT;
     const size_t bytes = (size_t)b->S.ncell * b->S.nq * sizeof(double);
     fill_guards(b);
-    k_soa_to_aos<<<grid_for(b->S.ncell), kThreads, 0, b->stream>>>(b->Pa, b->U, b->G);
+    launch_transpose<false>(b->Pa, b->U, b->G, b->stream);
     HIP_TRY(hipGetLastError());
     if (bytes >= THRESHOLD)
     {
@@ -1425,11 +1425,11 @@ extern "C" int mara_advance_noalloc(const mara_desc* d, const double* P_in, doub
     if (b.Pc) k_scratch_zero<<<zgrid, 256, 0, b.stream>>>(b.Pc, cellwords);
     if (b.Ssrc) k_scratch_zero<<<zgrid, 256, 0, b.stream>>>(b.Ssrc, cellwords);
     // MeshData::P -> the device layout, one step, and back
-    k_aos_to_soa<<<grid_for(b.S.ncell), kThreads, 0, b.stream>>>(P_in, b.Pa, b.G);
+    launch_transpose<true>(P_in, b.Pa, b.G, b.stream);
     k_ctl_begin_advance<<<1, 1, 0, b.stream>>>(b.ctl, dt);
     for (int rk = 0; rk < b.d.rk_order; ++rk) launch_stage(&b, rk, 0);
     fill_guards(&b);
-    k_soa_to_aos<<<grid_for(b.S.ncell), kThreads, 0, b.stream>>>(b.Pa, P_out, b.G);
+    launch_transpose<false>(b.Pa, P_out, b.G, b.stream);
     int status = MARA_OK;
     if (!hip_ok(hipGetLastError())) status = MARA_ERR_HIP;
     else if (!hip_ok(hipMemcpyAsync(&ctl_host, b.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, b.stream)))

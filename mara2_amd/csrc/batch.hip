@@ -631,7 +631,7 @@ int mara_batch_admit(mara_batch* B, const mara_desc* d, const double* P, double 
     // primitives: host -> staging (U) -> Pa, guards included; Pb starts as a copy
     if (!hip_ok(hipMemcpyAsync(it.U, P, sl.ncell * it.G.nq * sizeof(double), hipMemcpyHostToDevice, B->stream)))
         return undo();
-    k_aos_to_soa<<<(unsigned)((sl.ncell + 255) / 256), 256, 0, B->stream>>>(it.U, it.Pa, it.G);
+    launch_transpose<true>(it.U, it.Pa, it.G, B->stream);
     if (!hip_ok(hipMemcpyAsync(it.Pb, it.Pa, cb, hipMemcpyDeviceToDevice, B->stream))) return undo();
     if (it.S && !hip_ok(hipMemsetAsync(it.S, 0, cb, B->stream))) return undo();
     if (!hip_ok(hipGetLastError())) return undo();
@@ -862,7 +862,7 @@ int mara_batch_retire(mara_batch* B, int slot, double* P)
     BItem& it = B->items[slot];
     if (P)
     {
-        k_soa_to_aos<<<(unsigned)((sl.ncell + 255) / 256), 256, 0, B->stream>>>(it.Pa, it.U, it.G);
+        launch_transpose<false>(it.Pa, it.U, it.G, B->stream);
         HIP_TRY(hipMemcpyAsync(P, it.U, sl.ncell * it.G.nq * sizeof(double), hipMemcpyDeviceToHost, B->stream));
     }
     // the slot's control block stays inactive until the slot is reused: the
