@@ -851,7 +851,7 @@ int mara_block_upload_prim(mara_block* b, const double* P)
 {
     if (!b || !P) return MARA_ERR_INVALID_ARGUMENT;
     const size_t bytes = (size_t)b->S.ncell * b->S.nq * sizeof(double);
-    if (bytes >= THRESHOLD)
+    if (bytes >= UP_THRESHOLD)
     {
         HIP_TRY(hipStreamSynchronize(b->stream));
         HIP_TRY(copy_large(reinterpret_cast<char*>(b->U), reinterpret_cast<char*>(const_cast<double*>(P)), bytes, true));

@@ -11,8 +11,10 @@
 // 67.7 -> 16.1 ms, upload 25.1 -> 14.8 ms; 92 MB 9.1 -> 2.3 and 3.4 -> 2.2 ms;
 // 12.6 MB 0.85 -> 0.46 ms.  Chunks of 1 and 4 MiB and a stream per lane are no
 // faster; one stream for all takes 18 % longer, and each stream costs a
-// millisecond or two to make.  Copies below THRESHOLD stay with the runtime
-// (5.6 MB takes 0.36 ms there, about what the threads would).
+// millisecond or two to make.  Downloads below THRESHOLD stay with the runtime
+// (5.6 MB takes 0.36 ms there, about what the threads would), and uploads
+// below UP_THRESHOLD: 12.3 MB takes 0.38 ms there, 0.45 ms by the threads, and
+// a block that is only uploaded to should not pay for the set.
 //
 // Pinned chunks and streams are kept for the next copy while any block
 // exists: at most KEEP sets (32 MiB) idle, all given back with the last block.
@@ -36,6 +38,7 @@ constexpr int LANES = 8;
 constexpr int STREAMS = 2;  // shared by the lanes
 constexpr size_t CHUNK = 2u << 20;
 constexpr size_t THRESHOLD = 8u << 20;
+constexpr size_t UP_THRESHOLD = 32u << 20;
 constexpr size_t KEEP = 2;
 
 struct LaneSet
