@@ -29,9 +29,9 @@ namespace mara {
 // Tile height TY = 4 * rows for the launch shape's rows (1, 2 or 4).  LDS per
 // work-group (PLM): binary64 46 / 80 / 147 KB; binary32, with its staged
 // stencil zones, 40 / 66 / 116 KB.  64 x 8
-// tiles are the default in both forms: at 2048^2 their stage takes 0.51 ms
-// (binary64) and 0.33 ms (binary32) against 0.60 / 0.35 ms for 64 x 4 and
-// 0.54 / 0.36 ms for 64 x 16 (one work-group per CU).
+// tiles are the default in both forms: at 2048^2 their stage takes 0.36 ms
+// (binary64) and 0.26 ms (binary32) against 0.42 / 0.36 ms for 64 x 4 and
+// 0.39 / 0.30 ms for 64 x 16 (one work-group per CU).
 constexpr int MHD_ROWS_DEFAULT = 2;
 inline constexpr int mhd_tile_height(int rows) { return 4 * rows; }
 
