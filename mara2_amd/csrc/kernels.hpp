@@ -260,6 +260,16 @@ __device__ __forceinline__ void face_flux_lr(const R* PL, const R* PR, const Geo
         hlle<R, NQ, A>(SL, SR, Fq);
 }
 
+// WENO5's value on the right (Right) or left edge of the zone of v0
+template <int Law, typename R, bool Right, typename A>
+__device__ __forceinline__ R weno_side(R vm2, R vm1, R v0, R vp1, R vp2)
+{
+    if constexpr (Law == 2 && sizeof(R) == 8)
+        return weno_edge<Right>(weno_weights(vm2, vm1, v0, vp1, vp2), vm2, vm1, v0, vp1, vp2);
+    else
+        return weno5<R, Right, A>(vm2, vm1, v0, vp1, vp2);
+}
+
 // Flux through one face from its stencil S[q][m] = P(first stencil zone + m),
 // m = 0 .. 2 NG - 1, in R (reconstruction, law state, Riemann solver).
 template <int Law, int Recon, int Riem, typename R, typename A = LawMath<Law, R>, int AX = -1>
@@ -301,8 +311,8 @@ __device__ __forceinline__ void face_flux(const R (&S)[LawNQ<Law>::value][2 * St
         }
         else
         {
-            PL[q] = weno5<R, true, A>(S[q][0], S[q][1], S[q][2], S[q][3], S[q][4]);
-            PR[q] = weno5<R, false, A>(S[q][1], S[q][2], S[q][3], S[q][4], S[q][5]);
+            PL[q] = weno_side<Law, R, true, A>(S[q][0], S[q][1], S[q][2], S[q][3], S[q][4]);
+            PR[q] = weno_side<Law, R, false, A>(S[q][1], S[q][2], S[q][3], S[q][4], S[q][5]);
         }
     }
     face_flux_lr<Law, Riem, R, A, AX>(PL, PR, G, axis, Fq, ctlw);
@@ -333,8 +343,8 @@ __device__ __forceinline__ void face_flux_at(const double* __restrict__ P, const
             R v[6];
 #pragma unroll
             for (int m = 0; m < 6; ++m) v[m] = R(Pq[m * stride]);
-            PL[q] = weno5<R, true, A>(v[0], v[1], v[2], v[3], v[4]);
-            PR[q] = weno5<R, false, A>(v[1], v[2], v[3], v[4], v[5]);
+            PL[q] = weno_side<Law, R, true, A>(v[0], v[1], v[2], v[3], v[4]);
+            PR[q] = weno_side<Law, R, false, A>(v[1], v[2], v[3], v[4], v[5]);
             asm volatile("" : : "v"(PL[q]), "v"(PR[q]) : "memory");
         }
         face_flux_lr<Law, Riem, R, A, AX>(PL, PR, G, axis, Fq, ctlw);

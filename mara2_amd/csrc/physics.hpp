@@ -169,12 +169,13 @@ __device__ __forceinline__ R plm(R theta, R vl, R v0, R vr, R sgnv)
     return v0 + sgnv * R(0.5) * minmod<R, A>(theta, vl, v0, vr);
 }
 
-// WENO5 in the relativistic law's and the fast form's binary64: what a zone's
-// two edges share (each candidate's 1 / e_k^2, multiplied through by all three
-// e^2, so that one reciprocal serves the three and another their weighted sum)
-// and one edge from it.  The products stay far from the exponent range's ends,
-// scaled by the largest indicator, for any state the law's inversion accepts
-// (Z < 1e20).  Contractions are written out: a face gives the same value
+// WENO5 in the relativistic law's binary64: what a zone's two edges share (each
+// candidate's 1 / e_k^2, multiplied through by all three e^2, so that one
+// reciprocal serves the three and another their weighted sum) and one edge
+// from it.  Scaled by the largest indicator the products stay far from the
+// exponent range's ends for any state the law's inversion accepts (Z < 1e20);
+// the fast binary64 form of the other laws, which takes any state, keeps
+// weno5 (jumps beyond 1e70 would leave that range).  Contractions are written out: a face gives the same value
 // whether its zones' weights were shared or not.  Two reciprocals in place of
 // five: relativistic flux sweep at 128^3, 211 -> 205 us.
 struct WenoWeights
@@ -227,8 +228,6 @@ __device__ __forceinline__ double weno_edge(const WenoWeights& W, double vm2, do
 template <typename R, bool Right, typename D = Math<R>>
 __device__ __forceinline__ R weno5(R vm2, R vm1, R v0, R vp1, R vp2)
 {
-    if constexpr (sizeof(R) == 8 && D::ieee_minmax)
-        return weno_edge<Right>(weno_weights(vm2, vm1, v0, vp1, vp2), vm2, vm1, v0, vp1, vp2);
     // coefficient rows c[r][0..2] and weights d[r]
     const R c00 = Right ? R(1. / 3.) : R(11. / 6.), c01 = Right ? R(5. / 6.) : R(-7. / 6.), c02 = Right ? R(-1. / 6.) : R(1. / 3.);
     const R c10 = Right ? R(-1. / 6.) : R(1. / 3.), c11 = R(5. / 6.), c12 = Right ? R(1. / 3.) : R(-1. / 6.);
